@@ -231,6 +231,17 @@ int upload_eos_table(const HostEos &H, void **dev_pc, void **dev_tt, EosTable &T
   T.f_last = (float)T.e_last;
   T.f_inv_first_span = (float)T.inv_first_span;
   T.f_inv_last_span = (float)T.inv_last_span;
+  auto bits = [](auto x) {
+    typename std::conditional<sizeof(x) == 8, unsigned long long, unsigned>::type u;
+    std::memcpy(&u, &x, sizeof u);
+    return u;
+  };
+  T.hi_first = (unsigned)(bits(T.e_first) >> 32);
+  T.hi_span = (unsigned)(bits(T.e_pen) >> 32) - T.hi_first;
+  if (T.M >= 1 << 24) T.hi_span = 0;  // the lookup multiplies 24-bit integers
+  T.fb_first = bits(T.f_first);
+  // an e_0 below the normal FP32 numbers leaves the FP32 lookup its general path
+  T.fb_span = T.f_first >= 1.17549435e-38f && T.hi_span ? bits(T.f_pen) - T.fb_first : 0u;
   return GVH_OK;
 }
 

@@ -45,6 +45,9 @@ struct EosTable {
   double inv_first_span;     // 1/(e_1 - e_0)
   double inv_last_span;      // 1/(e_{n-1} - e_{n-2})
   float f_first, f_pen, f_last, f_inv_first_span, f_inv_last_span;  // the same in FP32
+  // high word (FP64) or bits (FP32) of e_0 = 2^emin_exp, and how far those of
+  // e_{n-2} lie above it: the range of the branch-free lookup
+  unsigned hi_first, hi_span, fb_first, fb_span;
 };
 
 struct StageArgs {
@@ -211,33 +214,29 @@ __device__ __forceinline__ double slope(double x, double y, double z) {
 // The IEEE-exact expansions of a/b and sqrt(x) on gfx950 cost ~11 and ~15
 // VALU instructions.  These start from the hardware approximations
 // (v_rcp_f64, v_rsq_f64: at most 4.6e-8 and 5.3e-8 relative, measured on
-// 4M inputs over [1e-6, 1e6]) and refine with FMA steps to 0.5 ulp on
-// those inputs (the reciprocal needs both Newton steps: one leaves 10 ulp).
-// Operands here are finite, normal and nonzero in any physical state;
-// special values are not treated.
+// 4M inputs over [1e-6, 1e6]) and refine with FMA steps.  A third-order step
+// takes the reciprocal to 0.5 ulp; a quotient and a square root end with a
+// residual correction, which needs its reciprocal only to 2e-15.  Operands
+// here are finite, normal and nonzero in any physical state; special values
+// are not treated, except that sqrt_nr(0) is 0 to within 1e-150.
 __device__ __forceinline__ double rcp_nr(double b) {
-  double r = __builtin_amdgcn_rcp(b);
-  double e = fma(-b, r, 1.0);
-  r = fma(r, e, r);
-  e = fma(-b, r, 1.0);
-  return fma(r, e, r);
+  const double r = __builtin_amdgcn_rcp(b);
+  const double e = fma(-b, r, 1.0);
+  return fma(r, fma(e, e, e), r);
 }
 __device__ __forceinline__ double div_nr(double a, double b) {
-  const double r = rcp_nr(b);
+  double r = __builtin_amdgcn_rcp(b);
+  r = fma(fma(-b, r, 1.0), r, r);
   const double q = a * r;
   return fma(fma(-b, q, a), r, q);
 }
 __device__ __forceinline__ double sqrt_nr(double x) {
+  x = fmax(x, 1e-300);
   const double y = __builtin_amdgcn_rsq(x);  // ~ 1/sqrt(x)
-  double g = x * y, h = 0.5 * y;
-  double e = fma(-g, h, 0.5);
-  g = fma(g, e, g);
-  h = fma(h, e, h);
-  e = fma(-g, h, 0.5);
-  g = fma(g, e, g);
-  h = fma(h, e, h);
-  const double d = fma(-g, g, x);
-  return x == 0.0 ? x : fma(d, h, g);
+  double g = x * y;
+  const double h = 0.5 * y;
+  g = fma(g, fma(-g, h, 0.5), g);
+  return fma(fma(-g, g, x), h, g);
 }
 
 // The same operations in the arithmetic type of a root-find: FP64 as above,
@@ -284,6 +283,106 @@ __device__ __forceinline__ TabPos tab_locate(const EosTable &T, double e) {
   return r;
 }
 
+// tab_locate in FP32.
+struct TabPosF {
+  int k;
+  float fr;
+};
+__device__ __forceinline__ TabPosF tab_locate_f(const EosTable &T, float e) {
+  TabPosF r;
+  if (e >= T.f_first && e < T.f_last) {
+    int E;
+    const float m = frexpf(e, &E);
+    const float f = (2.0f * m - 1.0f) * (float)T.M;
+    const int j = (int)f;
+    r.fr = f - (float)j;
+    r.k = (E - 1 - T.emin_exp) * T.M + j;
+    if (r.k > T.n - 2) {
+      r.k = T.n - 2;
+      r.fr += 1.0f;
+    }
+  } else if (e >= T.f_last) {
+    r.k = T.n - 2;
+    r.fr = (e - T.f_pen) * T.f_inv_last_span;
+  } else {
+    r.k = 0;
+    r.fr = (e - T.f_first) * T.f_inv_first_span;
+  }
+  return r;
+}
+// Positions of N energy densities at once: the octave and the place in it come straight from the exponent and mantissa bits, with
+// one wave-wide test that all N lie in [e_0, e_{n-2}) and the general lookup
+// behind it: 9 VALU instructions per lookup instead of 24, the same node
+// and fraction.  Only lanes with an energy density outside that range take
+// the general position.
+template <int N>
+__device__ __forceinline__ void tab_locate_n(const EosTable &T, const double *e, unsigned *k,
+                                             double *fr) {
+  unsigned d[N], far = 0;
+  const double M = (double)T.M;
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    const unsigned hi = (unsigned)__double2hiint(e[n]);
+    d[n] = hi - T.hi_first;
+    far = d[n] > far ? d[n] : far;
+    const double f = fma(__builtin_amdgcn_frexp_mant(e[n]), M + M, -M);  // (2 m - 1) M
+    fr[n] = __builtin_amdgcn_fract(f);
+    k[n] = __umul24(d[n] >> 20, (unsigned)T.M) + (unsigned)(int)f;
+  }
+  if (__any(far >= T.hi_span)) {
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+      if (d[n] >= T.hi_span) {
+        const TabPos q = tab_locate(T, e[n]);
+        k[n] = (unsigned)q.k;
+        fr[n] = q.fr;
+      }
+  }
+}
+template <int N>
+__device__ __forceinline__ void tab_locate_n(const EosTable &T, const float *e, unsigned *k,
+                                             float *fr) {
+  unsigned d[N], far = 0;
+  const float M = (float)T.M;
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    const unsigned bits = __float_as_uint(e[n]);
+    d[n] = bits - T.fb_first;
+    far = d[n] > far ? d[n] : far;
+    const float x = fmaf(__builtin_amdgcn_frexp_mantf(e[n]), 2.0f, -1.0f), f = x * M;
+    fr[n] = fmaf(x, M, -truncf(f));
+    k[n] = __umul24(d[n] >> 23, (unsigned)T.M) + (unsigned)(int)f;
+  }
+  if (__any(far >= T.fb_span)) {
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+      if (d[n] >= T.fb_span) {
+        const TabPosF q = tab_locate_f(T, e[n]);
+        k[n] = (unsigned)q.k;
+        fr[n] = q.fr;
+      }
+  }
+}
+
+__device__ __forceinline__ TabPos tab_at(const EosTable &T, double e) {
+  unsigned k;
+  TabPos r;
+  tab_locate_n<1>(T, &e, &k, &r.fr);
+  r.k = (int)k;
+  return r;
+}
+
+// c[0] + c[1] x + ... by Horner's rule: one FMA per coefficient.  The WB fits
+// of the root-finds are bound by their FMAs; summed over explicit powers of
+// e they took 12 multiplications more per evaluation.
+template <int N>
+__device__ __forceinline__ double horner(const double (&c)[N], double x) {
+  double r = c[N - 1];
+#pragma unroll
+  for (int k = N - 2; k >= 0; --k) r = fma(r, x, c[k]);
+  return r;
+}
+
 // equilibriumPressure (EquationOfState.cu:31-80) and speedOfSoundSquared
 // (:83-116); the conformal c_s^2 is the reference's integer 1/3 == 0.
 template <int EOS>
@@ -293,44 +392,29 @@ __device__ __forceinline__ void eos_p_cs2(const EosTable &T, double e, double &p
     p = e / 3.0;
     cs2 = 0.0;
   } else if constexpr (EOS == EOS_TABLE) {
-    TabPos q = tab_locate(T, e);
+    const TabPos q = tab_at(T, e);
     const double4 v = ld_cell(T.pc, (unsigned)q.k);
     p = v.x + q.fr * v.y;
     cs2 = v.z + q.fr * v.w;
   } else {
-    double e2 = e * e, e3 = e2 * e, e4 = e3 * e, e5 = e4 * e, e6 = e5 * e;
-    double e7 = e6 * e, e8 = e7 * e, e9 = e8 * e, e10 = e9 * e, e11 = e10 * e;
-    double e12 = e11 * e, e13 = e12 * e;
-    double a = fma(1.9531729608963267e-11, e12, fma(3.1188455176941583e-7, e11,
-               fma(0.0009417586777847889, e10, fma(0.7158279081255019, e9,
-               fma(141.5073484468774, e8, fma(6340.448389300905, e7,
-               fma(41913.439282708554, e6, fma(334334.4309240126, e5,
-               fma(1.6357487344679043e6, e4, fma(3.1729694865420084e6, e3,
-               fma(1.077580993288114e6, e2, fma(9737.845799644809, e,
-               -0.25181736420168666))))))))))));
-    double b = fma(3.2581066229887368e-18, e12, fma(5.928138360995685e-11, e11,
-               fma(9.601103399348206e-7, e10, fma(0.002962497695527404, e9,
-               fma(2.3405487982094204, e8, fma(499.04919730607065, e7,
-               fma(26452.34905933697, e6, fma(278581.2989342773, e5,
-               fma(1.7851642641834426e6, e4, fma(1.3512402226067686e7, e3,
-               fma(2.0931169138134286e7, e2, fma(4.0574329080826794e6, e,
-               45829.44617893836))))))))))));
-    p = a / b;
-    double cn = 5.191934309650155e-32 + 4.123605749683891e-23 * e +
-                3.1955868410879504e-16 * e2 + 1.4170364808063119e-10 * e3 +
-                6.087136671592452e-6 * e4 + 0.02969737949090831 * e5 +
-                15.382615282179595 * e6 + 460.6487249985994 * e7 +
-                1612.4245252438795 * e8 + 275.0492627924299 * e9 +
-                58.60283714484669 * e10 + 6.504847576502024 * e11 +
-                0.03009027913262399 * e12 + 8.189430244031285e-6 * e13;
-    double cd = 1.4637868900982493e-30 + 6.716598285341542e-22 * e +
-                3.5477700458515908e-15 * e2 + 1.1225580509306008e-9 * e3 +
-                0.00003551782901018317 * e4 + 0.13653226327408863 * e5 +
-                60.85769171450653 * e6 + 1800.5461219450308 * e7 +
-                15190.225535036281 * e8 + 590.2572000057821 * e9 +
-                293.99144775704605 * e10 + 21.461303090563028 * e11 +
-                0.09301685073435291 * e12 + 0.000024810902623582917 * e13;
-    cs2 = cn / cd;
+    constexpr double pn[] = {-0.25181736420168666, 9737.845799644809, 1.077580993288114e6,
+        3.1729694865420084e6, 1.6357487344679043e6, 334334.4309240126, 41913.439282708554,
+        6340.448389300905, 141.5073484468774, 0.7158279081255019, 0.0009417586777847889,
+        3.1188455176941583e-7, 1.9531729608963267e-11};
+    constexpr double pd[] = {45829.44617893836, 4.0574329080826794e6, 2.0931169138134286e7,
+        1.3512402226067686e7, 1.7851642641834426e6, 278581.2989342773, 26452.34905933697,
+        499.04919730607065, 2.3405487982094204, 0.002962497695527404, 9.601103399348206e-7,
+        5.928138360995685e-11, 3.2581066229887368e-18};
+    p = div_nr(horner(pn, e), horner(pd, e));
+    constexpr double cn[] = {5.191934309650155e-32, 4.123605749683891e-23, 3.1955868410879504e-16,
+        1.4170364808063119e-10, 6.087136671592452e-6, 0.02969737949090831, 15.382615282179595,
+        460.6487249985994, 1612.4245252438795, 275.0492627924299, 58.60283714484669,
+        6.504847576502024, 0.03009027913262399, 8.189430244031285e-6};
+    constexpr double cd[] = {1.4637868900982493e-30, 6.716598285341542e-22, 3.5477700458515908e-15,
+        1.1225580509306008e-9, 0.00003551782901018317, 0.13653226327408863, 60.85769171450653,
+        1800.5461219450308, 15190.225535036281, 590.2572000057821, 293.99144775704605,
+        21.461303090563028, 0.09301685073435291, 0.000024810902623582917};
+    cs2 = div_nr(horner(cn, e), horner(cd, e));
   }
 }
 
@@ -339,7 +423,7 @@ __device__ __forceinline__ double eos_p(const EosTable &T, double e) {
   if constexpr (EOS == EOS_CONFORMAL) {
     return e / 3.0;
   } else if constexpr (EOS == EOS_TABLE) {
-    TabPos q = tab_locate(T, e);
+    const TabPos q = tab_at(T, e);
     const double4 v = ld_cell(T.pc, (unsigned)q.k);
     return v.x + q.fr * v.y;
   } else {
@@ -349,30 +433,12 @@ __device__ __forceinline__ double eos_p(const EosTable &T, double e) {
   }
 }
 
-// p and c_s^2 of the tabulated EoS in FP32 (tab_locate with float
-// arithmetic, FP32 node values).
+// p and c_s^2 of the table with FP32 node values.
 __device__ __forceinline__ void tab_p_cs2_f(const EosTable &T, float e, float &p, float &cs2) {
-  int k;
+  unsigned k;
   float fr;
-  if (e >= T.f_first && e < T.f_last) {
-    int E;
-    const float m = frexpf(e, &E);
-    const float f = (2.0f * m - 1.0f) * (float)T.M;
-    const int j = (int)f;
-    fr = f - (float)j;
-    k = (E - 1 - T.emin_exp) * T.M + j;
-    if (k > T.n - 2) {
-      k = T.n - 2;
-      fr += 1.0f;
-    }
-  } else if (e >= T.f_last) {
-    k = T.n - 2;
-    fr = (e - T.f_pen) * T.f_inv_last_span;
-  } else {
-    k = 0;
-    fr = (e - T.f_first) * T.f_inv_first_span;
-  }
-  const float4 v = ld_cell(T.pcf, (unsigned)k);
+  tab_locate_n<1>(T, &e, &k, &fr);
+  const float4 v = ld_cell(T.pcf, k);
   p = v.x + fr * v.y;
   cs2 = v.z + fr * v.w;
 }
@@ -410,25 +476,19 @@ __device__ __forceinline__ double eos_T(const EosTable &T, double e) {
   if constexpr (EOS == EOS_CONFORMAL) {
     return pow(e / EOS_FACTOR, 0.25);
   } else if constexpr (EOS == EOS_TABLE) {
-    TabPos q = tab_locate(T, e);
+    const TabPos q = tab_at(T, e);
     const double2 v = ld_cell(T.tt, (unsigned)q.k);
     return v.x + q.fr * v.y;
   } else {
-    double e2 = e * e, e3 = e2 * e, e4 = e3 * e, e5 = e4 * e, e6 = e5 * e;
-    double e7 = e6 * e, e8 = e7 * e, e9 = e8 * e, e10 = e9 * e, e11 = e10 * e;
-    double n = 1.510073201405604e-29 + 8.014062800678687e-18 * e +
-               2.4954778310451065e-10 * e2 + 0.000063810382643387 * e3 +
-               0.4873490574161924 * e4 + 207.48582344326206 * e5 +
-               6686.07424325115 * e6 + 14109.766109389702 * e7 +
-               1471.6180520527757 * e8 + 14.055788949565482 * e9 +
-               0.015421252394182246 * e10 + 1.5780479034557783e-6 * e11;
-    double d = 7.558667139355393e-28 + 1.3686372302041508e-16 * e +
-               2.998130743142826e-9 * e2 + 0.0005036835870305458 * e3 +
-               2.316902328874072 * e4 + 578.0778724946719 * e5 +
-               11179.193315394154 * e6 + 17965.67607192861 * e7 +
-               1051.0730543534657 * e8 + 5.916312075925817 * e9 +
-               0.003778342768228011 * e10 + 1.8472801679382593e-7 * e11;
-    return n / d;
+    constexpr double tn[] = {1.510073201405604e-29, 8.014062800678687e-18, 2.4954778310451065e-10,
+        0.000063810382643387, 0.4873490574161924, 207.48582344326206, 6686.07424325115,
+        14109.766109389702, 1471.6180520527757, 14.055788949565482, 0.015421252394182246,
+        1.5780479034557783e-6};
+    constexpr double td[] = {7.558667139355393e-28, 1.3686372302041508e-16, 2.998130743142826e-9,
+        0.0005036835870305458, 2.316902328874072, 578.0778724946719, 11179.193315394154,
+        17965.67607192861, 1051.0730543534657, 5.916312075925817, 0.003778342768228011,
+        1.8472801679382593e-7};
+    return div_nr(horner(tn, e), horner(td, e));
   }
 }
 
@@ -449,74 +509,134 @@ __device__ __forceinline__ float zeta_over_s(float T, float tpeak) {
 }
 
 // ------------------------------------------------------------ root-find
-// energyDensityFromConservedVariables, EnergyMomentumTensor.cu:19-48:
-// Newton on e with the caller's guess, stopping at |de| <= 1e-3 |e|; the
-// step is damped by 0.9 after MAX_ITERS/2 iterations.  The update
-// e0 - f/fp with fp = 1 - num/den is evaluated as e0 - f den/(den - num),
-// and 1/e0 is shared: three divisions per iteration instead of five, equal
-// to the reference's expression up to rounding.
-// One Newton update of e0 given p(e0) and c_s^2(e0).
-template <bool DAMPED, typename F>
-__device__ __forceinline__ bool newton_update(F &e0, F p, F cs2, F M0, F M, F Pi) {
-  const F ie0 = rcp_t(e0);
-  const F cst2 = p * ie0;
-  const F A = fma(M0, F(1) - cst2, Pi);
-  const F B = fma(M0, M0 + Pi, -M);
-  const F H = sqrt_t(fabs(A * A + F(4) * cst2 * B));
-  const F D = div_t(A - H, F(2) * cst2);
-  const F f = e0 + D;
-  const F dc = cs2 - cst2;
-  const F num = dc * (B + D * H - dc * cst2 * D * M0 * ie0);
-  const F den = cst2 * e0 * H;
-  const F step = div_t((DAMPED ? F(0.9) * f : f) * den, den - num);
-  const F e = e0 - step;
-  const bool done = fabs(e - e0) <= F(0.001) * fabs(e);
-  e0 = e;
-  return done;
-}
-template <int EOS, bool DAMPED, typename F = double>
-__device__ __forceinline__ bool newton_step(const EosTable &T, F &e0, F M0, F M, F Pi) {
-  F p, cs2;
-  eos_p_cs2_t<EOS, F>(T, e0, p, cs2);
-  return newton_update<DAMPED, F>(e0, p, cs2, M0, M, Pi);
-}
-
-// max_iters <= MAX_ITERS bounds the iterations (the reference: MAX_ITERS);
-// the damping still starts at MAX_ITERS/2.
-template <int EOS>
-__device__ __forceinline__ double solve_e(const EosTable &T, double ePrev, double M0,
-                                          double M, double Pi,
-                                          unsigned long long *diag, int max_iters) {
-  if constexpr (EOS == EOS_CONFORMAL) {
-    return fabs(sqrt(fabs(4.0 * M0 * M0 - 3.0 * M)) - M0);
+// ------------------------------------------------ lookups of a root-find
+// p and c_s^2, or p alone, of N energy densities.
+template <int EOS, int N, typename F>
+__device__ __forceinline__ void eos_p_cs2_n(const EosTable &T, const F *e, F *p, F *cs2) {
+  if constexpr (EOS == EOS_TABLE) {
+    unsigned k[N];
+    F fr[N];
+    tab_locate_n<N>(T, e, k, fr);
+    if constexpr (std::is_same<F, double>::value) {
+      double4 v[N];
+#pragma unroll
+      for (int n = 0; n < N; ++n) v[n] = ld_cell(T.pc, k[n]);
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        p[n] = v[n].x + fr[n] * v[n].y;
+        cs2[n] = v[n].z + fr[n] * v[n].w;
+      }
+    } else {
+      float4 v[N];
+#pragma unroll
+      for (int n = 0; n < N; ++n) v[n] = ld_cell(T.pcf, k[n]);
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        p[n] = v[n].x + fr[n] * v[n].y;
+        cs2[n] = v[n].z + fr[n] * v[n].w;
+      }
+    }
   } else {
-    // A NaN iterate never meets the stopping rule and every later iterate is
-    // NaN, so the reference's 10^6 iterations end on NaN: leaving at the
-    // first NaN returns the same value.
-    double e = ePrev;
-    bool nan = false;
-    const int lim1 = max_iters < MAX_ITERS / 2 ? max_iters : MAX_ITERS / 2;
-    for (int it = 0; it < lim1 && !nan; ++it) {
-      if (newton_step<EOS, false>(T, e, M0, M, Pi)) return e;
-      nan = isnan(e);
+#pragma unroll
+    for (int n = 0; n < N; ++n) eos_p_cs2_t<EOS, F>(T, e[n], p[n], cs2[n]);
+  }
+}
+template <int EOS, int N, typename F>
+__device__ __forceinline__ void eos_p_n(const EosTable &T, const F *e, F *p) {
+  if constexpr (EOS == EOS_TABLE) {
+    unsigned k[N];
+    F fr[N];
+    tab_locate_n<N>(T, e, k, fr);
+    if constexpr (std::is_same<F, double>::value) {
+      double2 v[N];
+#pragma unroll
+      for (int n = 0; n < N; ++n) v[n] = ld_cell(reinterpret_cast<const double2 *>(T.pc), 2 * k[n]);
+#pragma unroll
+      for (int n = 0; n < N; ++n) p[n] = v[n].x + fr[n] * v[n].y;
+    } else {
+      float2 v[N];
+#pragma unroll
+      for (int n = 0; n < N; ++n) v[n] = ld_cell(reinterpret_cast<const float2 *>(T.pcf), 2 * k[n]);
+#pragma unroll
+      for (int n = 0; n < N; ++n) p[n] = v[n].x + fr[n] * v[n].y;
     }
-    for (int it = MAX_ITERS / 2; it < max_iters && !nan; ++it) {
-      if (newton_step<EOS, true>(T, e, M0, M, Pi)) return e;
-      nan = isnan(e);
-    }
-    atomicAdd(&diag[DIAG_NOT_CONVERGED], 1ull);
-    return e;  // the last iterate, as the reference returns e0 after e0 = e
+  } else {
+#pragma unroll
+    for (int n = 0; n < N; ++n) p[n] = eos_p_t<EOS, F>(T, e[n]);
   }
 }
 
-// N independent root-finds sharing the guess ePrev, run in lockstep: every
-// iteration evaluates all N Newton steps without branches and a chain keeps
-// its iterate once it has converged, so each result equals solve_e's for
-// that chain.  A wave already iterates until its slowest lane converges, so
-// the instruction count matches N sequential solves while the N table
-// gathers and dependency chains overlap.
+// What a Newton step needs of the iterate e0 alone.
+template <typename F>
+struct NewtonAt {
+  F p, w, om, dc, vi;  // p, w = p/e0, 1 - w, c_s^2 - w, (c_s^2 - w) w/e0
+};
+template <typename F>
+__device__ __forceinline__ NewtonAt<F> newton_at(F e0, F p, F cs2) {
+  NewtonAt<F> g;
+  const F ie0 = rcp_t(e0);
+  g.p = p;
+  g.w = p * ie0;
+  g.om = F(1) - g.w;
+  g.dc = cs2 - g.w;
+  g.vi = g.dc * g.w * ie0;
+  return g;
+}
+
+// Newton step of one root-find (EnergyMomentumTensor.cu:22-44).  With w =
+// p/e0, A = M0 (1 - w) + Pi, B = M0 (M0 + Pi) - M, H = sqrt|A^2 + 4 w B| and
+// D = (A - H)/(2 w) the reference takes f = e0 + D and f' = 1 - num/(w e0 H),
+// num = (c_s^2 - w)(B + D H - (c_s^2 - w) w D M0/e0).  Multiplied through by
+// w the quotient has one division instead of three,
+//   f/f' = p H (p + d) / (w p H - (c_s^2 - w)(w B + d (H - (c_s^2 - w) w M0/e0))),
+// d = w D = (A - H)/2: equal up to rounding, and the halving is exact.
+template <typename F>
+__device__ __forceinline__ F newton_step(const NewtonAt<F> &g, F M0, F B, F Pi) {
+  const F a = fma(M0, g.om, Pi);
+  const F q = g.w * B;
+  const F h = sqrt_t(fabs(fma(F(4), q, a * a)));
+  const F d = F(0.5) * (a - h);
+  const F y = fma(d, fma(-g.vi, M0, h), q);
+  const F ph = g.p * h;
+  return div_t(ph * (g.p + d), fma(-g.dc, y, g.w * ph));
+}
+
+// The guess of a cell's root-finds: its own energy density with p and c_s^2
+// there.  The cell's own inversion and its 12 half-site ones all start from
+// it, so the first iteration of each takes them from here.
+template <typename F>
+struct Guess {
+  F e, p, cs2;
+};
+template <int EOS, typename F>
+__device__ __forceinline__ Guess<F> make_guess(const EosTable &T, F e) {
+  Guess<F> g;
+  g.e = e;
+  g.p = g.cs2 = F(0);
+  if constexpr (EOS != EOS_CONFORMAL) eos_p_cs2_n<EOS, 1, F>(T, &g.e, &g.p, &g.cs2);
+  return g;
+}
+
+// energyDensityFromConservedVariables (EnergyMomentumTensor.cu:19-48) for N
+// root-finds that share the guess, in lockstep: Newton on e, stopping at
+// |de| <= 1e-3 |e|, the step damped by 0.9 after MAX_ITERS/2 iterations.
+// max_iters <= MAX_ITERS bounds the iterations (the reference: MAX_ITERS).
+// Every iteration evaluates all N steps without branches and a chain keeps
+// its iterate once it has converged, so each result equals that of a
+// root-find of its own, while the table gathers and the dependency chains of
+// the N overlap.  The loop is the wave's: it ends when no lane has a chain
+// left.  A NaN iterate never meets the reference's stopping rule and every
+// later one is NaN, so its 10^6 iterations return NaN: the chain stops there
+// and is counted as not converged.
+//
+// The first iteration is apart from the loop, since its p and c_s^2 are the
+// guess's: no lookup, and 1/e0 and the terms of NewtonAt once for all N.  On
+// a 201x201x101 lattice with every cell on this branch the FP64 stage kernel
+// issues 5100 VALU instructions per wave against 6450 with three divisions per
+// step, the general lookup in every iteration and a divergent loop: 2.05
+// against 2.34 ms per step.
 template <int EOS, int N, typename F = double>
-__device__ __forceinline__ void solve_e_lockstep(const EosTable &T, F ePrev, const F *M0,
+__device__ __forceinline__ void solve_e_lockstep(const EosTable &T, const Guess<F> &g, const F *M0,
                                                  const F *M, const F *Pi, F *e,
                                                  unsigned long long *diag, int max_iters) {
   if constexpr (EOS == EOS_CONFORMAL) {
@@ -526,50 +646,65 @@ __device__ __forceinline__ void solve_e_lockstep(const EosTable &T, F ePrev, con
       e[k] = fabs((std::is_same<F, double>::value ? sqrt(r) : sqrt_t(r)) - M0[k]);
     }
   } else {
-    unsigned act = (1u << N) - 1u;
+    F B[N];
+    bool live[N], any = false;
 #pragma unroll
-    for (int k = 0; k < N; ++k) e[k] = ePrev;
-    unsigned failed = 0;  // chains that reached a NaN iterate (see solve_e)
-    const int lim1 = max_iters < MAX_ITERS / 2 ? max_iters : MAX_ITERS / 2;
-    for (int it = 0; it < lim1 && act; ++it) {
-      // the N table gathers first, all in flight together
-      F pk[N], ck[N];
-#pragma unroll
-      for (int k = 0; k < N; ++k) eos_p_cs2_t<EOS, F>(T, e[k], pk[k], ck[k]);
+    for (int k = 0; k < N; ++k) {
+      B[k] = fma(M0[k], M0[k] + Pi[k], -M[k]);
+      e[k] = g.e;
+      live[k] = true;
+    }
+    // the scheduler would mix the first steps into the code before them and
+    // run out of registers
+    __builtin_amdgcn_sched_barrier(0);
+    if (max_iters > 0) {
+      const NewtonAt<F> at = newton_at(g.e, g.p, g.cs2);
 #pragma unroll
       for (int k = 0; k < N; ++k) {
-        F ek = e[k];
-        const bool done = newton_update<false, F>(ek, pk[k], ck[k], M0[k], M[k], Pi[k]);
-        const bool live = (act >> k) & 1u;
-        e[k] = live ? ek : e[k];
-        if (live && done) act &= ~(1u << k);
-        if (live && !done && isnan(ek)) {
-          act &= ~(1u << k);
-          failed |= 1u << k;
-        }
+        const F step = newton_step(at, M0[k], B[k], Pi[k]);
+        e[k] = g.e - step;
+        // a NaN step compares false and ends the chain
+        live[k] = fabs(step) > F(0.001) * fabs(e[k]);
+        any = any || live[k];
       }
     }
-    for (int it = MAX_ITERS / 2; it < max_iters && act; ++it) {
-      // the N table gathers first, all in flight together
-      F pk[N], ck[N];
-#pragma unroll
-      for (int k = 0; k < N; ++k) eos_p_cs2_t<EOS, F>(T, e[k], pk[k], ck[k]);
+    __builtin_amdgcn_sched_barrier(0);
+    F scale = F(1), tol = F(0.001);  // of the step; tol = 0.001 / scale
+    for (int it = 1; it < max_iters && __builtin_amdgcn_ballot_w64(any); ++it) {
+      if (it == MAX_ITERS / 2) {
+        scale = F(0.9);
+        tol = F(0.001 / 0.9);
+      }
+      F p[N], cs2[N];
+      eos_p_cs2_n<EOS, N, F>(T, e, p, cs2);
+      any = false;
 #pragma unroll
       for (int k = 0; k < N; ++k) {
-        F ek = e[k];
-        const bool done = newton_update<true, F>(ek, pk[k], ck[k], M0[k], M[k], Pi[k]);
-        const bool live = (act >> k) & 1u;
-        e[k] = live ? ek : e[k];
-        if (live && done) act &= ~(1u << k);
-        if (live && !done && isnan(ek)) {
-          act &= ~(1u << k);
-          failed |= 1u << k;
-        }
+        const F step = newton_step(newton_at(e[k], p[k], cs2[k]), M0[k], B[k], Pi[k]);
+        const F ek = fma(-scale, step, e[k]);
+        e[k] = live[k] ? ek : e[k];
+        live[k] = live[k] && fabs(step) > tol * fabs(ek);
+        any = any || live[k];
       }
     }
-    act |= failed;
-    if (act) atomicAdd(&diag[DIAG_NOT_CONVERGED], (unsigned long long)__popc(act));
+#pragma unroll
+    for (int k = 0; k < N; ++k) any = any || isnan(e[k]);
+    if (any) {
+      int bad = 0;
+#pragma unroll
+      for (int k = 0; k < N; ++k) bad += (live[k] || isnan(e[k])) ? 1 : 0;
+      atomicAdd(&diag[DIAG_NOT_CONVERGED], (unsigned long long)bad);
+    }
   }
+}
+
+template <int EOS>
+__device__ __forceinline__ double solve_e(const EosTable &T, const Guess<double> &g, double M0,
+                                          double M, double Pi, unsigned long long *diag,
+                                          int max_iters) {
+  double e;
+  solve_e_lockstep<EOS, 1, double>(T, g, &M0, &M, &Pi, &e, diag, max_iters);
+  return e;
 }
 
 struct Prim {
@@ -582,12 +717,12 @@ template <int EOS>
 __device__ __forceinline__ Prim inferred(const EosTable &T, double t, double ttt,
                                          double ttx, double tty, double ttn,
                                          double pitt, double pitx, double pity,
-                                         double pitn, double Pi, double ePrev,
+                                         double pitn, double Pi, const Guess<double> &g,
                                          unsigned long long *diag, int max_iters) {
   double M0 = ttt - pitt, M1 = ttx - pitx, M2 = tty - pity, M3 = ttn - pitn;
   double M = M1 * M1 + M2 * M2 + t * t * M3 * M3;
   Prim r;
-  r.e = (ePrev <= 0.1) ? M0 - M / M0 : solve_e<EOS>(T, ePrev, M0, M, Pi, diag, max_iters);
+  r.e = (g.e <= 0.1) ? M0 - M / M0 : solve_e<EOS>(T, g, M0, M, Pi, diag, max_iters);
   if (isnan(r.e)) atomicAdd(&diag[DIAG_E_NAN], 1ull);
   r.p = eos_p<EOS>(T, r.e);
   if (r.e < 1.e-7) {
@@ -615,11 +750,11 @@ template <int EOS, int DIR>
 __device__ __forceinline__ double flux_velocity(const EosTable &T, double t, double ttt,
                                                 double ttx, double tty, double ttn, double pitt,
                                                 double pitx, double pity, double pitn,
-                                                double Pi, double ePrev,
+                                                double Pi, const Guess<double> &g,
                                                 unsigned long long *diag, int max_iters) {
   const double M0 = ttt - pitt, M1 = ttx - pitx, M2 = tty - pity, M3 = ttn - pitn;
   const double M = M1 * M1 + M2 * M2 + t * t * M3 * M3;
-  double e = (ePrev <= 0.1) ? M0 - M / M0 : solve_e<EOS>(T, ePrev, M0, M, Pi, diag, max_iters);
+  double e = (g.e <= 0.1) ? M0 - M / M0 : solve_e<EOS>(T, g, M0, M, Pi, diag, max_iters);
   if (isnan(e)) atomicAdd(&diag[DIAG_E_NAN], 1ull);
   double p = eos_p<EOS>(T, e);
   if (e < 1.e-7) {
@@ -633,7 +768,8 @@ __device__ __forceinline__ double flux_velocity(const EosTable &T, double t, dou
 }
 
 // flux_velocity of N half-site states of one direction that share the
-// guess ePrev, with their root-finds in lockstep (solve_e_lockstep).
+// guess g, with their root-finds in lockstep (solve_e_lockstep); vacuum: the
+// guess is at most 0.1 fm^-4, where the reference takes the closed form.
 // W[k] = (T^tt, T^tx, T^ty, T^tn, pi^tt, pi^tx, pi^ty, pi^tn, Pi).
 // In the mixed form (R = float) the root-finds of the flux states run in FP32
 // for the conformal and tabulated EoS: their results only set the flux
@@ -647,7 +783,8 @@ using flux_root_t =
 
 template <int EOS, int DIR, int N, typename R, bool ROOT64 = false>
 __device__ __forceinline__ void flux_velocity_lockstep(const EosTable &T, double t,
-                                                       const R (*W)[9], double ePrev,
+                                                       const R (*W)[9], bool vacuum,
+                                                       const Guess<flux_root_t<EOS, R, ROOT64>> &g,
                                                        unsigned long long *diag, int max_iters,
                                                        double *v) {
   using F = flux_root_t<EOS, R, ROOT64>;
@@ -662,29 +799,35 @@ __device__ __forceinline__ void flux_velocity_lockstep(const EosTable &T, double
     Md[k] = DIR == 0 ? M1 : (DIR == 1 ? M2 : M3);
     Pi[k] = (F)W[k][8];
   }
-  if (ePrev <= 0.1) {
+  if (vacuum) {
 #pragma unroll
     for (int k = 0; k < N; ++k) e[k] = M0[k] - div_t(M[k], M0[k]);
   } else {
-    solve_e_lockstep<EOS, N, F>(T, F(ePrev), M0, M, Pi, e, diag, max_iters);
+    solve_e_lockstep<EOS, N, F>(T, g, M0, M, Pi, e, diag, max_iters);
   }
-  // the N pressure gathers first, so that they are in flight together (an
-  // atomic between them would order them)
-  F pk[N];
+  F p[N];
+  eos_p_n<EOS, N, F>(T, e, p);
+  // NaN and clamped states are rare: one test for all N
+  bool plain = true;
 #pragma unroll
-  for (int k = 0; k < N; ++k) pk[k] = eos_p_t<EOS, F>(T, e[k]);
+  for (int k = 0; k < N; ++k) plain = plain && e[k] >= F(1.e-7);
+  if (!plain) {
+    int nan = 0, low = 0;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      nan += isnan(e[k]) ? 1 : 0;
+      if (e[k] < F(1.e-7)) {
+        e[k] = p[k] = F(1.e-7);
+        ++low;
+      }
+    }
+    if (nan) atomicAdd(&diag[DIAG_E_NAN], (unsigned long long)nan);
+    if (low) atomicAdd(&diag[DIAG_E_CLAMPED], (unsigned long long)low);
+  }
 #pragma unroll
   for (int k = 0; k < N; ++k) {
-    F ek = e[k];
-    if (isnan(ek)) atomicAdd(&diag[DIAG_E_NAN], 1ull);
-    F p = pk[k];
-    if (ek < F(1.e-7)) {
-      ek = F(1.e-7);
-      p = F(1.e-7);
-      atomicAdd(&diag[DIAG_E_CLAMPED], 1ull);
-    }
-    const F P = p + Pi[k];
-    v[k] = (double)div_t((ek + P > F(0)) ? Md[k] : -Md[k], fabs(M0[k] + P));
+    const F P = p[k] + Pi[k];
+    v[k] = (double)div_t((e[k] + P > F(0)) ? Md[k] : -Md[k], fabs(M0[k] + P));
   }
 }
 

@@ -60,7 +60,7 @@ using Grad = GradT<double>;
 // relaxation right-hand sides of pi^{mu nu} and Pi.
 template <int EOS, bool BULK, typename R>
 __device__ __forceinline__ void source_terms(const StageArgs &A, const R *Q, double e_eos,
-                                             R e, R p, R ut, R ux, R uy, R un, R utp, R uxp,
+                                             double cs2, R e, R p, R ut, R ux, R uy, R un, R utp, R uxp,
                                              R uyp, R unp, const GradT<R> &g, R *S) {
   const R t = R(A.t);
   const R inv_t = div_st(R(1.0), t);
@@ -246,12 +246,10 @@ __device__ __forceinline__ void source_terms(const StageArgs &A, const R *Q, dou
     S[13] = r * inv_ut + pinn * dkvk;
   }
   if constexpr (BULK) {
-    // bulk relaxation, :53-60 and :238, :254; c_s^2 from the FP64 EoS (1/3 -
+    // bulk relaxation, :53-60 and :238, :254; cs2 is the FP64 EoS's (1/3 -
     // c_s^2 is small where the fluid is nearly conformal), zeta/s in the
     // arithmetic of the source terms
     using FE = R;
-    double p_, cs2;
-    eos_p_cs2<EOS>(A.tab, e_eos, p_, cs2);
     const R a = R(0.333333f) - R(cs2);
     const R a2 = a * a;
     const R beta_Pi = R(15.0) * a2 * (e + p);
@@ -287,9 +285,9 @@ constexpr int BLOCK = GVH_BLOCK;
 // LDS copy of rows j-2 .. j+2 (ystage[variable][row slot][lane]) instead of
 // from memory.
 template <int EOS, bool BULK, int DIR, bool KEEP_STATES, int LOCK, typename R, typename PS,
-          bool YSTAGE = false>
+          bool YSTAGE = false, typename GF>
 __device__ __forceinline__ void direction_update(const StageArgs &A, unsigned s, double ePrev,
-                                                 R v_s, double *acc,
+                                                 const Guess<GF> &g, R v_s, double *acc,
                                                  const R *ystage = nullptr) {
   constexpr int NV = BULK ? 15 : 14;
   const long long st = DIR == 0 ? 1 : (DIR == 1 ? (long long)A.ncx : (long long)A.ncx * A.ncy);
@@ -305,12 +303,10 @@ __device__ __forceinline__ void direction_update(const StageArgs &A, unsigned s,
   auto ldp = [&](int n, long long o) -> R { return R(ld_cell(qP + (n - 4) * G + o, s)); };
 
   // the six spatial pi components, whose flux comes after that of the kept
-  // states: their 30 stencil values in one batch.  In FP32 they are loaded
-  // before the root-finds and stay in flight during them; in FP64 the 60
-  // registers this takes would cost a wave per SIMD, so they are loaded
-  // after the root-finds.
+  // states: their 30 stencil values in one batch, after the root-finds.  In
+  // flight during them they would cost a wave per SIMD in FP64 and spills in
+  // FP32 (1.55 against 1.48 ms per step on the 201x201x101 lattice).
   constexpr bool FLUX_FROM_KEPT = KEEP_STATES && LOCK != 2;
-  constexpr bool EARLY_RAW2 = FLUX_FROM_KEPT && sizeof(R) == 4;
   R raw2[6][5];
   auto load_raw2 = [&]() {
 #pragma unroll
@@ -355,18 +351,17 @@ __device__ __forceinline__ void direction_update(const StageArgs &A, unsigned s,
       Wst[3][a] = vm1 + half_slope_t<R>(vm2, vm1, v0);
       if (a >= 4) cdv[a - 4] = (vp1 - vm1) * hc;
     }
-    if constexpr (EARLY_RAW2) load_raw2();
     double v4[4];
     if constexpr (LOCK) {
-      flux_velocity_lockstep<EOS, DIR, 4, R, LOCK == 3>(A.tab, t, Wst, ePrev, A.diag,
-                                                        A.max_iters, v4);
+      flux_velocity_lockstep<EOS, DIR, 4, R, LOCK == 3>(A.tab, t, Wst, ePrev <= 0.1, g,
+                                                        A.diag, A.max_iters, v4);
     } else {
 #pragma unroll
       for (int k = 0; k < 4; ++k)
         v4[k] = flux_velocity<EOS, DIR>(A.tab, t, (double)Wst[k][0], (double)Wst[k][1],
                                         (double)Wst[k][2], (double)Wst[k][3], (double)Wst[k][4],
                                         (double)Wst[k][5], (double)Wst[k][6], (double)Wst[k][7],
-                                        (double)Wst[k][8], ePrev, A.diag, A.max_iters);
+                                        (double)Wst[k][8], g, A.diag, A.max_iters);
     }
     vRf = v4[0];
     vLf = v4[1];
@@ -392,7 +387,7 @@ __device__ __forceinline__ void direction_update(const StageArgs &A, unsigned s,
       }
       const double v = flux_velocity<EOS, DIR>(A.tab, t, (double)w[0], (double)w[1], (double)w[2],
                                                (double)w[3], (double)w[4], (double)w[5],
-                                               (double)w[6], (double)w[7], (double)w[8], ePrev,
+                                               (double)w[6], (double)w[7], (double)w[8], g,
                                                A.diag, A.max_iters);
       vRf = state == 0 ? v : vRf;
       vLf = state == 1 ? v : vLf;
@@ -415,7 +410,7 @@ __device__ __forceinline__ void direction_update(const StageArgs &A, unsigned s,
   const R aB = fmax(fabs(rLb), fabs(rRb));
 
 
-  if constexpr (FLUX_FROM_KEPT && !EARLY_RAW2) load_raw2();
+  if constexpr (FLUX_FROM_KEPT) load_raw2();
 
   // directional sources: central differences of pi^{tau mu} and Pi and of
   // the three spatial pi components of this direction
@@ -575,7 +570,7 @@ __global__ __launch_bounds__(BLOCK) void kt_source_kernel(StageArgs A) {
   for (int n = 0; n < 15; ++n) Q[n] = (n < NV) ? (A.qin + n * G)[s] : 0.0;
   S[14] = 0.0;
   const double *up = A.uprev;
-  source_terms<EOS, BULK, double>(A, Q, e_s, e_s, p_s, ut, ux, uy, un, up[s], (up + G)[s],
+  source_terms<EOS, BULK, double>(A, Q, e_s, make_guess<EOS>(A.tab, e_s).cs2, e_s, p_s, ut, ux, uy, un, up[s], (up + G)[s],
                                   (up + 2 * G)[s], (up + 3 * G)[s], g, S);
 #pragma unroll
   for (int n = 0; n < NV; ++n) (A.qout + n * G)[s] = Q[n] + A.dt * S[n];
@@ -608,12 +603,20 @@ __device__ __forceinline__ void stage_cell(const StageArgs &A, const CellPos &c,
   };
   const double *u = A.uin;
   double ut = 1.0, ux = 0.0, uy = 0.0, un = 0.0, e_s = 0.0;
+  // the root-finds' guess: the half-site ones' in their arithmetic (FP64
+  // where they run one at a time), the cell's own in FP64
+  using GF = typename std::conditional<LOCK != 0, flux_root_t<EOS, R, LOCK == 3>, double>::type;
+  Guess<double> guess{};
+  Guess<GF> fguess{};
   if (!YSTAGE || c.valid) {
     ut = ld_cell(u, s);
     ux = ld_cell(u + G, s);
     uy = ld_cell(u + 2 * G, s);
     un = ld_cell(u + 3 * G, s);
     e_s = ld_cell(A.ein, s);
+    guess = make_guess<EOS>(A.tab, e_s);
+    if constexpr (std::is_same<GF, double>::value) fguess = guess;
+    else fguess = make_guess<EOS>(A.tab, GF(e_s));
     if constexpr (FUSED) {
       const double p_s = ld_cell(A.pin, s);
       GradT<R> g;
@@ -641,7 +644,7 @@ __device__ __forceinline__ void stage_cell(const StageArgs &A, const CellPos &c,
       }
       S[14] = R(0);
       const double *up = A.uprev;
-      source_terms<EOS, BULK, R>(A, Q, e_s, R(e_s), R(p_s), R(ut), R(ux), R(uy), R(un),
+      source_terms<EOS, BULK, R>(A, Q, e_s, guess.cs2, R(e_s), R(p_s), R(ut), R(ux), R(uy), R(un),
                                  R(ld_cell(up, s)), R(ld_cell(up + G, s)),
                                  R(ld_cell(up + 2 * G, s)), R(ld_cell(up + 3 * G, s)), g, S);
 #pragma unroll
@@ -652,15 +655,17 @@ __device__ __forceinline__ void stage_cell(const StageArgs &A, const CellPos &c,
     }
 
     // flux velocity of the cell itself for the directional sources (v = u/u^tau)
-    direction_update<EOS, BULK, 0, KEEP, LOCK, R, PS>(A, s, e_s, div_st(R(ux), R(ut)), acc);
+    direction_update<EOS, BULK, 0, KEEP, LOCK, R, PS>(A, s, e_s, fguess, div_st(R(ux), R(ut)),
+                                                       acc);
   }
   if constexpr (YSTAGE) {
     __syncthreads();
     if (!c.valid) return;
   }
-  direction_update<EOS, BULK, 1, KEEP, LOCK, R, PS, YSTAGE>(A, s, e_s, div_st(R(uy), R(ut)), acc,
-                                                            ystage);
-  if constexpr (HAS_Z) direction_update<EOS, BULK, 2, KEEP, LOCK, R, PS>(A, s, e_s, div_st(R(un), R(ut)), acc);
+  direction_update<EOS, BULK, 1, KEEP, LOCK, R, PS, YSTAGE>(A, s, e_s, fguess, div_st(R(uy), R(ut)),
+                                                            acc, ystage);
+  if constexpr (HAS_Z)
+    direction_update<EOS, BULK, 2, KEEP, LOCK, R, PS>(A, s, e_s, fguess, div_st(R(un), R(ut)), acc);
 
   if constexpr (STAGE2) {
     // q^n of the convex average: all NV loads in flight together
@@ -674,7 +679,9 @@ __device__ __forceinline__ void stage_cell(const StageArgs &A, const CellPos &c,
   // inferred variables with this cell's e as the guess
   const Prim pr = inferred<EOS>(A.tab, A.tinf, acc[0], acc[BLOCK], acc[2 * BLOCK], acc[3 * BLOCK],
                                 acc[4 * BLOCK], acc[5 * BLOCK], acc[6 * BLOCK], acc[7 * BLOCK],
-                                BULK ? acc[14 * BLOCK] : 0.0, e_s, A.diag, A.max_iters);
+                                BULK ? acc[14 * BLOCK] : 0.0,
+                                sizeof(R) == 8 ? guess : make_guess<EOS>(A.tab, e_s), A.diag,
+                                A.max_iters);
 
   // regulateDissipativeCurrents (RegulateDissipativeCurrents.cu:16-134): only
   // cells at or below e_reg are rescaled; the bulk factor is 1 unless p is 0.
