@@ -299,6 +299,9 @@ extern "C" int gvh_create(const gvh_lattice_parameters *lattice, const gvh_hydro
   e = hipMemsetAsync(c->arena, 0, bytes, c->stream);
   if (e == hipSuccess) e = hipMalloc((void **)&c->diag, DIAG_N * sizeof(unsigned long long));
   if (e == hipSuccess) e = hipMalloc((void **)&c->count, sizeof(unsigned long long));
+  if (e == hipSuccess) e = hipMalloc((void **)&c->tickets, RESIDENT_TICKETS * sizeof(unsigned));
+  if (e == hipSuccess)
+    e = hipMemsetAsync(c->tickets, 0, RESIDENT_TICKETS * sizeof(unsigned), c->stream);
   if (e == hipSuccess) e = hipMemsetAsync(c->diag, 0, DIAG_N * sizeof(unsigned long long), c->stream);
   if (e == hipSuccess) e = hipEventCreate(&c->ev[0]);
   if (e == hipSuccess) e = hipEventCreate(&c->ev[1]);
@@ -344,6 +347,7 @@ extern "C" int gvh_destroy(gvh_context *c) {
   if (c->arena) (void)hipFree(c->arena);
   if (c->diag) (void)hipFree(c->diag);
   if (c->count) (void)hipFree(c->count);
+  if (c->tickets) (void)hipFree(c->tickets);
   if (c->tab_pc) (void)hipFree(c->tab_pc);
   if (c->tab_tt) (void)hipFree(c->tab_tt);
   if (c->validity) (void)hipFree(c->validity);
@@ -557,6 +561,7 @@ StageArgs make_stage_args(gvh_context *c, int stage, double t) {
   StageArgs A{};
   stage_pointers(A, context_buffers(c), context_roles(c), stage);
   A.diag = c->diag;
+  A.tickets = c->tickets;
   A.reg = (stage == 2 && c->validity) ? c->validity + GVH_V_REGULATIONS * c->G : nullptr;
   A.G = c->G;
   A.nx = c->nx;
@@ -580,6 +585,7 @@ StageArgs make_stage_args(gvh_context *c, int stage, double t) {
   A.tab = c->tab;
   A.strip = c->strip;
   A.nstrips = (c->ny + c->strip - 1) / c->strip;
+  A.ntiles = (unsigned)((((long long)c->nx * c->strip * A.nstrips * c->nz + 63) / 64 + 7) / 8 * 8);
   A.variant = c->variant;
   A.max_iters = c->max_iters;
   return A;

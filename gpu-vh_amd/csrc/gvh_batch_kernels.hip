@@ -29,7 +29,7 @@ __global__ __launch_bounds__(BLOCK, stage_waves_per_simd<R>()) void kt_batch_ker
   stage_times(A, S.t0 + S.steps * S.A.dt, STAGE2 ? 2 : 1);
   const CellPos c = cell_of_tile(A, (unsigned)(t - S.tile_first), (unsigned)S.ntiles);
   if (c.valid)
-    stage_cell<EOS, BULK, STAGE2, HAS_Z, true, KEEP, LOCK, R, PS>(A, c, acc_lds + threadIdx.x);
+    stage_cell<EOS, BULK, STAGE2, HAS_Z, true, KEEP, LOCK, R, PS>(A, A.tab, c, acc_lds + threadIdx.x);
 }
 
 // The run loop's per-step history update (FreezeOut.cpp:49-126) for every

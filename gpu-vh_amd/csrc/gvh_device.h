@@ -29,6 +29,19 @@ enum { EOS_CONFORMAL = 0, EOS_WB = 1, EOS_TABLE = 2 };
 #define GVH_BLOCK 64
 #endif
 
+// Lattices of at least this many tiles of 64 cells run their stages in the
+// resident kernel (gvh_resident.hip).  Its blocks start with a copy of the
+// table and its 2048 (FP64) or 3072 waves end together only if each has
+// several tiles.  us per step, one-wave blocks against resident, table EoS
+// with bulk: 101x101x31 (4941 tiles) 208 / 219 FP64 and 138 / 145 mixed,
+// 101x101x51 (8129) 311 / 308 and 202 / 205, 151x151x41 (14607) 540 / 527
+// and 380 / 352, 201x201x101 (63757) 2120 / 2040 and 1469 / 1332.
+#ifndef GVH_RESIDENT_MIN_TILES
+#define GVH_RESIDENT_MIN_TILES 10240
+#endif
+constexpr unsigned RESIDENT_MIN_TILES = GVH_RESIDENT_MIN_TILES;
+constexpr int RESIDENT_TICKETS = 512;  // its tile counters, 32-bit words
+
 // counters of failure events, indexes into StageArgs::diag
 enum { DIAG_NOT_CONVERGED = 0, DIAG_E_NAN = 1, DIAG_E_CLAMPED = 2, DIAG_N = 4 };
 
@@ -62,6 +75,7 @@ struct StageArgs {
   double *__restrict__ eout;
   double *__restrict__ pout;
   unsigned long long *__restrict__ diag;
+  unsigned *__restrict__ tickets;  // tile counters of the resident kernel (gvh_resident.hip)
   double *__restrict__ reg;  // stage 2 stores the shear regulation factor here if set
   long long G;          // stride between variables
   int nx, ny, nz, ncx, ncy;
@@ -74,6 +88,7 @@ struct StageArgs {
   double e_reg;         // regulation below this energy density
   EosTable tab;
   int strip, nstrips;   // y rows per traversal strip, number of strips
+  unsigned ntiles;      // blocks of 64 cells of the traversal, a multiple of 8
   int variant;          // kernel arrangement of a stage (gvh_stage.hip)
   int max_iters;        // Newton iterations per root-find: MAX_ITERS (the reference's),
                         // or a smaller budget of a batched event
@@ -364,6 +379,55 @@ __device__ __forceinline__ void tab_locate_n(const EosTable &T, const float *e, 
   }
 }
 
+// Node k: {p_k, p_{k+1} - p_k, cs2_k, cs2_{k+1} - cs2_k} (tab_pc), its first
+// half (tab_pp) and {T_k, T_{k+1} - T_k} (tab_tt).
+__device__ __forceinline__ double4 tab_pc(const EosTable &T, unsigned k) { return ld_cell(T.pc, k); }
+__device__ __forceinline__ double2 tab_pp(const EosTable &T, unsigned k) {
+  return ld_cell(reinterpret_cast<const double2 *>(T.pc), 2 * k);
+}
+__device__ __forceinline__ double2 tab_tt(const EosTable &T, unsigned k) { return ld_cell(T.tt, k); }
+__device__ __forceinline__ float4 tab_pcf(const EosTable &T, unsigned k) { return ld_cell(T.pcf, k); }
+__device__ __forceinline__ float2 tab_ppf(const EosTable &T, unsigned k) {
+  return ld_cell(reinterpret_cast<const float2 *>(T.pcf), 2 * k);
+}
+
+// The table with copies of its nodes in LDS.  FP64 nodes are either whole
+// (WIDE: as in T.pc) or {p_k, cs2_k}, whose differences are taken at the
+// lookup (the same subtraction of the same values as in T.pc); FP32 nodes are
+// as in T.pcf.  T(e) stays in memory: one lookup per cell and stage.
+constexpr int TAB_LDS_NODES = 2048;
+template <bool WIDE>
+struct LdsTable : EosTable {
+  const double2 *n64;
+  const float4 *n32;
+  __device__ __forceinline__ LdsTable(const EosTable &T, const double2 *a, const float4 *b)
+      : EosTable(T), n64(a), n32(b) {}
+};
+template <bool WIDE>
+__device__ __forceinline__ double4 tab_pc(const LdsTable<WIDE> &T, unsigned k) {
+  if constexpr (WIDE) {
+    const double2 a = T.n64[2 * k], b = T.n64[2 * k + 1];
+    return double4{a.x, a.y, b.x, b.y};
+  } else {
+    const double2 a = T.n64[k], b = T.n64[k + 1];
+    return double4{a.x, b.x - a.x, a.y, b.y - a.y};
+  }
+}
+template <bool WIDE>
+__device__ __forceinline__ double2 tab_pp(const LdsTable<WIDE> &T, unsigned k) {
+  if constexpr (WIDE) return T.n64[2 * k];
+  const double a = T.n64[k].x, b = T.n64[k + 1].x;
+  return double2{a, b - a};
+}
+template <bool WIDE>
+__device__ __forceinline__ float4 tab_pcf(const LdsTable<WIDE> &T, unsigned k) {
+  return T.n32[k];
+}
+template <bool WIDE>
+__device__ __forceinline__ float2 tab_ppf(const LdsTable<WIDE> &T, unsigned k) {
+  return *reinterpret_cast<const float2 *>(T.n32 + k);
+}
+
 __device__ __forceinline__ TabPos tab_at(const EosTable &T, double e) {
   unsigned k;
   TabPos r;
@@ -385,15 +449,15 @@ __device__ __forceinline__ double horner(const double (&c)[N], double x) {
 
 // equilibriumPressure (EquationOfState.cu:31-80) and speedOfSoundSquared
 // (:83-116); the conformal c_s^2 is the reference's integer 1/3 == 0.
-template <int EOS>
-__device__ __forceinline__ void eos_p_cs2(const EosTable &T, double e, double &p,
+template <int EOS, typename Tab>
+__device__ __forceinline__ void eos_p_cs2(const Tab &T, double e, double &p,
                                           double &cs2) {
   if constexpr (EOS == EOS_CONFORMAL) {
     p = e / 3.0;
     cs2 = 0.0;
   } else if constexpr (EOS == EOS_TABLE) {
     const TabPos q = tab_at(T, e);
-    const double4 v = ld_cell(T.pc, (unsigned)q.k);
+    const double4 v = tab_pc(T, (unsigned)q.k);
     p = v.x + q.fr * v.y;
     cs2 = v.z + q.fr * v.w;
   } else {
@@ -418,13 +482,13 @@ __device__ __forceinline__ void eos_p_cs2(const EosTable &T, double e, double &p
   }
 }
 
-template <int EOS>
-__device__ __forceinline__ double eos_p(const EosTable &T, double e) {
+template <int EOS, typename Tab>
+__device__ __forceinline__ double eos_p(const Tab &T, double e) {
   if constexpr (EOS == EOS_CONFORMAL) {
     return e / 3.0;
   } else if constexpr (EOS == EOS_TABLE) {
     const TabPos q = tab_at(T, e);
-    const double4 v = ld_cell(T.pc, (unsigned)q.k);
+    const double2 v = tab_pp(T, (unsigned)q.k);
     return v.x + q.fr * v.y;
   } else {
     double p, c;
@@ -434,19 +498,20 @@ __device__ __forceinline__ double eos_p(const EosTable &T, double e) {
 }
 
 // p and c_s^2 of the table with FP32 node values.
-__device__ __forceinline__ void tab_p_cs2_f(const EosTable &T, float e, float &p, float &cs2) {
+template <typename Tab>
+__device__ __forceinline__ void tab_p_cs2_f(const Tab &T, float e, float &p, float &cs2) {
   unsigned k;
   float fr;
   tab_locate_n<1>(T, &e, &k, &fr);
-  const float4 v = ld_cell(T.pcf, k);
+  const float4 v = tab_pcf(T, k);
   p = v.x + fr * v.y;
   cs2 = v.z + fr * v.w;
 }
 
 // eos_p_cs2 / eos_p in the arithmetic type F (float only for the conformal
 // and tabulated EoS).
-template <int EOS, typename F>
-__device__ __forceinline__ void eos_p_cs2_t(const EosTable &T, F e, F &p, F &cs2) {
+template <int EOS, typename F, typename Tab>
+__device__ __forceinline__ void eos_p_cs2_t(const Tab &T, F e, F &p, F &cs2) {
   if constexpr (std::is_same<F, double>::value) {
     eos_p_cs2<EOS>(T, e, p, cs2);
   } else {
@@ -459,8 +524,8 @@ __device__ __forceinline__ void eos_p_cs2_t(const EosTable &T, F e, F &p, F &cs2
     }
   }
 }
-template <int EOS, typename F>
-__device__ __forceinline__ F eos_p_t(const EosTable &T, F e) {
+template <int EOS, typename F, typename Tab>
+__device__ __forceinline__ F eos_p_t(const Tab &T, F e) {
   if constexpr (std::is_same<F, double>::value) {
     return eos_p<EOS>(T, e);
   } else {
@@ -471,13 +536,13 @@ __device__ __forceinline__ F eos_p_t(const EosTable &T, F e) {
 }
 
 // effectiveTemperature, EquationOfState.cu:119-148
-template <int EOS>
-__device__ __forceinline__ double eos_T(const EosTable &T, double e) {
+template <int EOS, typename Tab>
+__device__ __forceinline__ double eos_T(const Tab &T, double e) {
   if constexpr (EOS == EOS_CONFORMAL) {
     return pow(e / EOS_FACTOR, 0.25);
   } else if constexpr (EOS == EOS_TABLE) {
     const TabPos q = tab_at(T, e);
-    const double2 v = ld_cell(T.tt, (unsigned)q.k);
+    const double2 v = tab_tt(T, (unsigned)q.k);
     return v.x + q.fr * v.y;
   } else {
     constexpr double tn[] = {1.510073201405604e-29, 8.014062800678687e-18, 2.4954778310451065e-10,
@@ -511,8 +576,8 @@ __device__ __forceinline__ float zeta_over_s(float T, float tpeak) {
 // ------------------------------------------------------------ root-find
 // ------------------------------------------------ lookups of a root-find
 // p and c_s^2, or p alone, of N energy densities.
-template <int EOS, int N, typename F>
-__device__ __forceinline__ void eos_p_cs2_n(const EosTable &T, const F *e, F *p, F *cs2) {
+template <int EOS, int N, typename F, typename Tab>
+__device__ __forceinline__ void eos_p_cs2_n(const Tab &T, const F *e, F *p, F *cs2) {
   if constexpr (EOS == EOS_TABLE) {
     unsigned k[N];
     F fr[N];
@@ -520,7 +585,7 @@ __device__ __forceinline__ void eos_p_cs2_n(const EosTable &T, const F *e, F *p,
     if constexpr (std::is_same<F, double>::value) {
       double4 v[N];
 #pragma unroll
-      for (int n = 0; n < N; ++n) v[n] = ld_cell(T.pc, k[n]);
+      for (int n = 0; n < N; ++n) v[n] = tab_pc(T, k[n]);
 #pragma unroll
       for (int n = 0; n < N; ++n) {
         p[n] = v[n].x + fr[n] * v[n].y;
@@ -529,7 +594,7 @@ __device__ __forceinline__ void eos_p_cs2_n(const EosTable &T, const F *e, F *p,
     } else {
       float4 v[N];
 #pragma unroll
-      for (int n = 0; n < N; ++n) v[n] = ld_cell(T.pcf, k[n]);
+      for (int n = 0; n < N; ++n) v[n] = tab_pcf(T, k[n]);
 #pragma unroll
       for (int n = 0; n < N; ++n) {
         p[n] = v[n].x + fr[n] * v[n].y;
@@ -541,8 +606,8 @@ __device__ __forceinline__ void eos_p_cs2_n(const EosTable &T, const F *e, F *p,
     for (int n = 0; n < N; ++n) eos_p_cs2_t<EOS, F>(T, e[n], p[n], cs2[n]);
   }
 }
-template <int EOS, int N, typename F>
-__device__ __forceinline__ void eos_p_n(const EosTable &T, const F *e, F *p) {
+template <int EOS, int N, typename F, typename Tab>
+__device__ __forceinline__ void eos_p_n(const Tab &T, const F *e, F *p) {
   if constexpr (EOS == EOS_TABLE) {
     unsigned k[N];
     F fr[N];
@@ -550,13 +615,13 @@ __device__ __forceinline__ void eos_p_n(const EosTable &T, const F *e, F *p) {
     if constexpr (std::is_same<F, double>::value) {
       double2 v[N];
 #pragma unroll
-      for (int n = 0; n < N; ++n) v[n] = ld_cell(reinterpret_cast<const double2 *>(T.pc), 2 * k[n]);
+      for (int n = 0; n < N; ++n) v[n] = tab_pp(T, k[n]);
 #pragma unroll
       for (int n = 0; n < N; ++n) p[n] = v[n].x + fr[n] * v[n].y;
     } else {
       float2 v[N];
 #pragma unroll
-      for (int n = 0; n < N; ++n) v[n] = ld_cell(reinterpret_cast<const float2 *>(T.pcf), 2 * k[n]);
+      for (int n = 0; n < N; ++n) v[n] = tab_ppf(T, k[n]);
 #pragma unroll
       for (int n = 0; n < N; ++n) p[n] = v[n].x + fr[n] * v[n].y;
     }
@@ -608,8 +673,8 @@ template <typename F>
 struct Guess {
   F e, p, cs2;
 };
-template <int EOS, typename F>
-__device__ __forceinline__ Guess<F> make_guess(const EosTable &T, F e) {
+template <int EOS, typename F, typename Tab>
+__device__ __forceinline__ Guess<F> make_guess(const Tab &T, F e) {
   Guess<F> g;
   g.e = e;
   g.p = g.cs2 = F(0);
@@ -635,8 +700,8 @@ __device__ __forceinline__ Guess<F> make_guess(const EosTable &T, F e) {
 // issues 5100 VALU instructions per wave against 6450 with three divisions per
 // step, the general lookup in every iteration and a divergent loop: 2.05
 // against 2.34 ms per step.
-template <int EOS, int N, typename F = double>
-__device__ __forceinline__ void solve_e_lockstep(const EosTable &T, const Guess<F> &g, const F *M0,
+template <int EOS, int N, typename F, typename Tab>
+__device__ __forceinline__ void solve_e_lockstep(const Tab &T, const Guess<F> &g, const F *M0,
                                                  const F *M, const F *Pi, F *e,
                                                  unsigned long long *diag, int max_iters) {
   if constexpr (EOS == EOS_CONFORMAL) {
@@ -698,8 +763,8 @@ __device__ __forceinline__ void solve_e_lockstep(const EosTable &T, const Guess<
   }
 }
 
-template <int EOS>
-__device__ __forceinline__ double solve_e(const EosTable &T, const Guess<double> &g, double M0,
+template <int EOS, typename Tab>
+__device__ __forceinline__ double solve_e(const Tab &T, const Guess<double> &g, double M0,
                                           double M, double Pi, unsigned long long *diag,
                                           int max_iters) {
   double e;
@@ -713,8 +778,8 @@ struct Prim {
 
 // getInferredVariables, EnergyMomentumTensor.cu:51-108 (the '#ifdef Pi'
 // consistency fix at :82-85 is never compiled in the reference; omitted)
-template <int EOS>
-__device__ __forceinline__ Prim inferred(const EosTable &T, double t, double ttt,
+template <int EOS, typename Tab>
+__device__ __forceinline__ Prim inferred(const Tab &T, double t, double ttt,
                                          double ttx, double tty, double ttn,
                                          double pitt, double pitx, double pity,
                                          double pitn, double Pi, const Guess<double> &g,
@@ -746,8 +811,8 @@ __device__ __forceinline__ Prim inferred(const EosTable &T, double t, double ttt
 // u^tau = sqrt|(M0+P)E| and u_dir = M_dir E/u^tau, so
 // v = M_dir E/|(M0+P)E| = sign(e+P) M_dir/|M0+P|: one division and no square
 // root, equal up to rounding wherever e+P is finite and nonzero.
-template <int EOS, int DIR>
-__device__ __forceinline__ double flux_velocity(const EosTable &T, double t, double ttt,
+template <int EOS, int DIR, typename Tab>
+__device__ __forceinline__ double flux_velocity(const Tab &T, double t, double ttt,
                                                 double ttx, double tty, double ttn, double pitt,
                                                 double pitx, double pity, double pitn,
                                                 double Pi, const Guess<double> &g,
@@ -781,8 +846,8 @@ template <int EOS, typename R, bool ROOT64 = false>
 using flux_root_t =
     typename std::conditional<(sizeof(R) == 4 && EOS != EOS_WB && !ROOT64), float, double>::type;
 
-template <int EOS, int DIR, int N, typename R, bool ROOT64 = false>
-__device__ __forceinline__ void flux_velocity_lockstep(const EosTable &T, double t,
+template <int EOS, int DIR, int N, typename R, bool ROOT64, typename Tab>
+__device__ __forceinline__ void flux_velocity_lockstep(const Tab &T, double t,
                                                        const R (*W)[9], bool vacuum,
                                                        const Guess<flux_root_t<EOS, R, ROOT64>> &g,
                                                        unsigned long long *diag, int max_iters,

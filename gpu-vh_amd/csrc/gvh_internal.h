@@ -92,6 +92,7 @@ struct gvh_context {
   double *pbuf[2] = {nullptr, nullptr};
   unsigned long long *diag = nullptr;
   unsigned long long *count = nullptr;
+  unsigned *tickets = nullptr;  // tile counters of the resident stage kernel
 
   int iq = 0;   // buffer holding q^n
   int iu = 0;   // buffer holding u^n

@@ -5,6 +5,10 @@
 
 namespace gvh {
 
+bool resident_stage_fits(const StageArgs &A);
+hipError_t launch_resident_stage(const StageArgs &A, bool bulk, bool stage2, int precision,
+                                 hipStream_t st);
+
 // ------------------------------------------------------------ launch
 // Kernel arrangement of a stage (StageArgs::variant): 0 fused kernel with
 // the inversion states kept in registers, 1 fused with states rebuilt one at
@@ -116,6 +120,8 @@ static hipError_t launch_p(const StageArgs &A, int eos, bool bulk, bool stage2, 
 // precision: GVH_FP64, GVH_MIXED or GVH_MIXED_F64_ROOTS
 hipError_t launch_stage(const StageArgs &A, int eos, bool bulk, bool stage2, int precision,
                         hipStream_t st) {
+  if (A.variant == 3 && eos == EOS_TABLE && resident_stage_fits(A))
+    return launch_resident_stage(A, bulk, stage2, precision, st);
   if (precision == GVH_FP64) return launch_p<false>(A, eos, bulk, stage2, false, st);
   return launch_p<true>(A, eos, bulk, stage2, precision == GVH_MIXED_F64_ROOTS, st);
 }

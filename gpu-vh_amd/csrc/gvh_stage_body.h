@@ -58,8 +58,8 @@ using Grad = GradT<double>;
 // loadSourceTerms2 (SourceTerms.cu:570-755) with setPimunuSourceTerms
 // (:30-256): T^{tau mu} geometric and pressure-gradient sources and the
 // relaxation right-hand sides of pi^{mu nu} and Pi.
-template <int EOS, bool BULK, typename R>
-__device__ __forceinline__ void source_terms(const StageArgs &A, const R *Q, double e_eos,
+template <int EOS, bool BULK, typename R, typename Tab>
+__device__ __forceinline__ void source_terms(const StageArgs &A, const Tab &tab, const R *Q, double e_eos,
                                              double cs2, R e, R p, R ut, R ux, R uy, R un, R utp, R uxp,
                                              R uyp, R unp, const GradT<R> &g, R *S) {
   const R t = R(A.t);
@@ -84,7 +84,7 @@ __device__ __forceinline__ void source_terms(const StageArgs &A, const R *Q, dou
   S[3] = -R(3.0) * Q[3] * inv_t - g.p[2] * inv_t2 + dkvk * pitn;
 
   // transport coefficients, SourceTerms.cu:46-60
-  const double T_eos = eos_T<EOS>(A.tab, e_eos);
+  const double T_eos = eos_T<EOS>(tab, e_eos);
   const R T = R(T_eos);
   const R taupiInv = R(0.2f) * div_st(T, R(A.etabar));
   const R beta_pi = R(0.2f) * (e + p);
@@ -285,8 +285,8 @@ constexpr int BLOCK = GVH_BLOCK;
 // LDS copy of rows j-2 .. j+2 (ystage[variable][row slot][lane]) instead of
 // from memory.
 template <int EOS, bool BULK, int DIR, bool KEEP_STATES, int LOCK, typename R, typename PS,
-          bool YSTAGE = false, typename GF>
-__device__ __forceinline__ void direction_update(const StageArgs &A, unsigned s, double ePrev,
+          bool YSTAGE = false, typename Tab, typename GF>
+__device__ __forceinline__ void direction_update(const StageArgs &A, const Tab &tab, unsigned s, double ePrev,
                                                  const Guess<GF> &g, R v_s, double *acc,
                                                  const R *ystage = nullptr) {
   constexpr int NV = BULK ? 15 : 14;
@@ -353,12 +353,12 @@ __device__ __forceinline__ void direction_update(const StageArgs &A, unsigned s,
     }
     double v4[4];
     if constexpr (LOCK) {
-      flux_velocity_lockstep<EOS, DIR, 4, R, LOCK == 3>(A.tab, t, Wst, ePrev <= 0.1, g,
+      flux_velocity_lockstep<EOS, DIR, 4, R, LOCK == 3>(tab, t, Wst, ePrev <= 0.1, g,
                                                         A.diag, A.max_iters, v4);
     } else {
 #pragma unroll
       for (int k = 0; k < 4; ++k)
-        v4[k] = flux_velocity<EOS, DIR>(A.tab, t, (double)Wst[k][0], (double)Wst[k][1],
+        v4[k] = flux_velocity<EOS, DIR>(tab, t, (double)Wst[k][0], (double)Wst[k][1],
                                         (double)Wst[k][2], (double)Wst[k][3], (double)Wst[k][4],
                                         (double)Wst[k][5], (double)Wst[k][6], (double)Wst[k][7],
                                         (double)Wst[k][8], g, A.diag, A.max_iters);
@@ -385,7 +385,7 @@ __device__ __forceinline__ void direction_update(const StageArgs &A, unsigned s,
         const R xm = ld(n, o - st), x0 = ld(n, o), xp = ld(n, o + st);
         w[a] = x0 + half_slope_t<R>(xm, x0, xp) * sg;
       }
-      const double v = flux_velocity<EOS, DIR>(A.tab, t, (double)w[0], (double)w[1], (double)w[2],
+      const double v = flux_velocity<EOS, DIR>(tab, t, (double)w[0], (double)w[1], (double)w[2],
                                                (double)w[3], (double)w[4], (double)w[5],
                                                (double)w[6], (double)w[7], (double)w[8], g,
                                                A.diag, A.max_iters);
@@ -510,10 +510,8 @@ struct CellPos {
 // The thread index and its quotients are 32-bit: a lattice's ghosted cell
 // count is below 2^29 (every array of 8-byte values is below 4 GiB), and the
 // grid exceeds the cell count by less than one strip plus 8 blocks.
-__device__ __forceinline__ CellPos cell_of_tile(const StageArgs &A, unsigned b, unsigned nb) {
-  const unsigned lb = (b & 7u) * (nb >> 3) + (b >> 3);
+__device__ __forceinline__ CellPos cell_of_index(const StageArgs &A, unsigned tid) {
   const unsigned by = (unsigned)A.strip, nx = (unsigned)A.nx, nz = (unsigned)A.nz;
-  const unsigned tid = lb * BLOCK + threadIdx.x;
   const unsigned r = tid / nx;
   const int i = (int)(tid - r * nx);
   const unsigned r2 = r / by;
@@ -529,6 +527,11 @@ __device__ __forceinline__ CellPos cell_of_tile(const StageArgs &A, unsigned b, 
   c.k = k + NG;
   c.s = (unsigned)c.i + (unsigned)A.ncx * ((unsigned)c.j + (unsigned)A.ncy * (unsigned)c.k);
   return c;
+}
+
+__device__ __forceinline__ CellPos cell_of_tile(const StageArgs &A, unsigned b, unsigned nb) {
+  const unsigned lb = (b & 7u) * (nb >> 3) + (b >> 3);
+  return cell_of_index(A, lb * BLOCK + threadIdx.x);
 }
 
 __device__ __forceinline__ CellPos cell_of_thread(const StageArgs &A) {
@@ -570,7 +573,7 @@ __global__ __launch_bounds__(BLOCK) void kt_source_kernel(StageArgs A) {
   for (int n = 0; n < 15; ++n) Q[n] = (n < NV) ? (A.qin + n * G)[s] : 0.0;
   S[14] = 0.0;
   const double *up = A.uprev;
-  source_terms<EOS, BULK, double>(A, Q, e_s, make_guess<EOS>(A.tab, e_s).cs2, e_s, p_s, ut, ux, uy, un, up[s], (up + G)[s],
+  source_terms<EOS, BULK, double>(A, A.tab, Q, e_s, make_guess<EOS>(A.tab, e_s).cs2, e_s, p_s, ut, ux, uy, un, up[s], (up + G)[s],
                                   (up + 2 * G)[s], (up + 3 * G)[s], g, S);
 #pragma unroll
   for (int n = 0; n < NV; ++n) (A.qout + n * G)[s] = Q[n] + A.dt * S[n];
@@ -587,8 +590,9 @@ __global__ __launch_bounds__(BLOCK) void kt_source_kernel(StageArgs A) {
 // direction, and only threads of valid cells compute (the others only
 // staged rows for their neighbours).
 template <int EOS, bool BULK, bool STAGE2, bool HAS_Z, bool FUSED, bool KEEP, int LOCK,
-          typename R, typename PS, bool YSTAGE = false>
-__device__ __forceinline__ void stage_cell(const StageArgs &A, const CellPos &c, double *acc,
+          typename R, typename PS, bool YSTAGE = false, typename Tab>
+__device__ __forceinline__ void stage_cell(const StageArgs &A, const Tab &tab, const CellPos &c,
+                                           double *acc,
                                            const R *ystage = nullptr) {
   constexpr int NV = BULK ? 15 : 14;
   const int i = c.i, j = c.j, k = c.k;
@@ -614,9 +618,9 @@ __device__ __forceinline__ void stage_cell(const StageArgs &A, const CellPos &c,
     uy = ld_cell(u + 2 * G, s);
     un = ld_cell(u + 3 * G, s);
     e_s = ld_cell(A.ein, s);
-    guess = make_guess<EOS>(A.tab, e_s);
+    guess = make_guess<EOS>(tab, e_s);
     if constexpr (std::is_same<GF, double>::value) fguess = guess;
-    else fguess = make_guess<EOS>(A.tab, GF(e_s));
+    else fguess = make_guess<EOS>(tab, GF(e_s));
     if constexpr (FUSED) {
       const double p_s = ld_cell(A.pin, s);
       GradT<R> g;
@@ -644,7 +648,7 @@ __device__ __forceinline__ void stage_cell(const StageArgs &A, const CellPos &c,
       }
       S[14] = R(0);
       const double *up = A.uprev;
-      source_terms<EOS, BULK, R>(A, Q, e_s, guess.cs2, R(e_s), R(p_s), R(ut), R(ux), R(uy), R(un),
+      source_terms<EOS, BULK, R>(A, tab, Q, e_s, guess.cs2, R(e_s), R(p_s), R(ut), R(ux), R(uy), R(un),
                                  R(ld_cell(up, s)), R(ld_cell(up + G, s)),
                                  R(ld_cell(up + 2 * G, s)), R(ld_cell(up + 3 * G, s)), g, S);
 #pragma unroll
@@ -655,17 +659,17 @@ __device__ __forceinline__ void stage_cell(const StageArgs &A, const CellPos &c,
     }
 
     // flux velocity of the cell itself for the directional sources (v = u/u^tau)
-    direction_update<EOS, BULK, 0, KEEP, LOCK, R, PS>(A, s, e_s, fguess, div_st(R(ux), R(ut)),
+    direction_update<EOS, BULK, 0, KEEP, LOCK, R, PS>(A, tab, s, e_s, fguess, div_st(R(ux), R(ut)),
                                                        acc);
   }
   if constexpr (YSTAGE) {
     __syncthreads();
     if (!c.valid) return;
   }
-  direction_update<EOS, BULK, 1, KEEP, LOCK, R, PS, YSTAGE>(A, s, e_s, fguess, div_st(R(uy), R(ut)),
+  direction_update<EOS, BULK, 1, KEEP, LOCK, R, PS, YSTAGE>(A, tab, s, e_s, fguess, div_st(R(uy), R(ut)),
                                                             acc, ystage);
   if constexpr (HAS_Z)
-    direction_update<EOS, BULK, 2, KEEP, LOCK, R, PS>(A, s, e_s, fguess, div_st(R(un), R(ut)), acc);
+    direction_update<EOS, BULK, 2, KEEP, LOCK, R, PS>(A, tab, s, e_s, fguess, div_st(R(un), R(ut)), acc);
 
   if constexpr (STAGE2) {
     // q^n of the convex average: all NV loads in flight together
@@ -677,10 +681,10 @@ __device__ __forceinline__ void stage_cell(const StageArgs &A, const CellPos &c,
   }
 
   // inferred variables with this cell's e as the guess
-  const Prim pr = inferred<EOS>(A.tab, A.tinf, acc[0], acc[BLOCK], acc[2 * BLOCK], acc[3 * BLOCK],
+  const Prim pr = inferred<EOS>(tab, A.tinf, acc[0], acc[BLOCK], acc[2 * BLOCK], acc[3 * BLOCK],
                                 acc[4 * BLOCK], acc[5 * BLOCK], acc[6 * BLOCK], acc[7 * BLOCK],
                                 BULK ? acc[14 * BLOCK] : 0.0,
-                                sizeof(R) == 8 ? guess : make_guess<EOS>(A.tab, e_s), A.diag,
+                                sizeof(R) == 8 ? guess : make_guess<EOS>(tab, e_s), A.diag,
                                 A.max_iters);
 
   // regulateDissipativeCurrents (RegulateDissipativeCurrents.cu:16-134): only
@@ -759,7 +763,7 @@ __global__ __launch_bounds__(BLOCK, (stage_waves_per_simd<R, LOCK>())) void kt_f
   __shared__ double acc_lds[15 * BLOCK];
   const CellPos c = cell_of_thread(A);
   if (!c.valid) return;
-  stage_cell<EOS, BULK, STAGE2, HAS_Z, FUSED, KEEP, LOCK, R, PS>(A, c, acc_lds + threadIdx.x);
+  stage_cell<EOS, BULK, STAGE2, HAS_Z, FUSED, KEEP, LOCK, R, PS>(A, A.tab, c, acc_lds + threadIdx.x);
 }
 
 // ------------------------------------- y stencil staged in LDS (arrangement 5)
@@ -832,7 +836,7 @@ kt_flux_kernel_ystaged(StageArgs A) {
       ystage[(a * 8 + slot) * BLOCK + lane] = in ? v : R(0);
     }
   }
-  stage_cell<EOS, BULK, STAGE2, HAS_Z, true, true, LOCK, R, PS, true>(A, cr.c, acc_lds[w] + lane,
+  stage_cell<EOS, BULK, STAGE2, HAS_Z, true, true, LOCK, R, PS, true>(A, A.tab, cr.c, acc_lds[w] + lane,
                                                                      ystage);
 }
 
