@@ -119,7 +119,7 @@ size_t event_footprint(const gvh_lattice_parameters &L, int precision, int surfa
     const size_t nrow = (size_t)fofreq * nx * ny;
     bytes += 2 * (size_t)(fofreq + 1) * 10 * nint * sizeof(double);  // ring, two halves
     bytes += 2 * nrow * sizeof(unsigned) * 5 / 4;                // row counts and offsets
-    bytes += nint / 20 * (3 * sizeof(unsigned) + 80 * sizeof(double) + 200 * sizeof(double));
+    bytes += nint / 20 * (4 * sizeof(unsigned) + 80 * sizeof(double) + 200 * sizeof(double));
   }
   return bytes;
 }

@@ -634,5 +634,454 @@ __device__ int cell_elements(Work &W, double (*cen)[D], double (*nrm)[D]) {
   return nh;
 }
 
+// ------------------------------------------------ plain cells, one per lane
+// A plain cell has no square with four cuts, no cube whose six lines are two
+// triangles, and polygons that are one polyhedron: nearly every cell of a
+// smooth surface.  Which lines it has, and the order in which the general
+// search lists them, then follow from the corner pattern alone:
+//  * a cube with three to five lines is one polygon, its lines in square
+//    order; one with six is a hexagon, followed from its first line around,
+//    turning lines whose end meets;
+//  * the polygons come in cube order, or, where a hexagon (or the 24-line
+//    pattern of two corners) makes the cell ambiguous, each time the first
+//    one that shares a square with those before it.
+// So a lane takes a whole cell: it lists its lines (a byte each), computes the
+// cut of each of the 32 edges once (the squares that share an edge cut it at
+// the same point) and goes over the list four times, summing in the general
+// search's order: the element equals its bit by bit.  End points are matched
+// by edge where the general search matches coordinates within 1e-10; cells
+// with a cut that near a corner are left to it.
+
+// Corner pattern of a cell (corner c = sum of side * 2^(d-1-axis)): bit c is
+// set where the value is at least v0.  False for values that are no number,
+// or so near v0 that the product of two differences could vanish.
+template <int NC>
+__device__ __forceinline__ bool corner_mask(const double *v, double v0, unsigned &above) {
+  bool odd = false;
+  above = 0;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const double d = v[c] - v0;
+    above |= (v[c] >= v0 ? 1u : 0u) << c;
+    odd = odd || !(fabs(d) >= 1e-140 || d == 0.0);
+  }
+  return !odd;
+}
+
+// Cut of the edge from value a to value b (exactly one of them below v0).
+__device__ __forceinline__ double edge_cut(double a, double b, double v0, double h) {
+  if (a == v0) return 1e-9 * h;
+  if (b == v0) return (1.0 - 1e-9) * h;
+  return (a - v0) / (a - b) * h;
+}
+
+// x / 3, correctly rounded: quotient by the rounded reciprocal and one
+// residual correction (Markstein).
+__device__ __forceinline__ double third(double x) {
+  const double r = 1.0 / 3.0, q = x * r;
+  return fma(fma(-3.0, q, x), r, q);
+}
+
+// Squares of a cell: number 6 q + r, q = 2 a + j the cube that holds axis a
+// at side j, r = 2 f + jj its square that holds the cube's f-th free axis at
+// side jj.  A 3-D cell is the cube q = 0 with corners 0..7.
+struct SquareInfo {
+  unsigned base, w1, w2;    // corner (0, 0); corner weights of the free axes
+  unsigned x1, x2, a, xf;   // free axes x1 < x2, held axes
+  unsigned j, jj;           // sides of a and xf
+  unsigned i0, i1, i2, i3;  // edges (x2 = 0), (x1 = 0), (x1 = h1), (x2 = h2)
+};
+// Edge number: axis * 8 + the corner's sides along the other axes.
+__device__ __forceinline__ unsigned edge_number(unsigned d, unsigned corner) {
+  return d * 8 + ((corner >> (4 - d)) << (3 - d) | (corner & ((8u >> d) - 1u)));
+}
+__device__ __forceinline__ uint2 pack_square(unsigned n) {
+  const unsigned q = n / 6, r = n - 6 * q, a = q >> 1, j = q & 1, f = r >> 1, jj = r & 1;
+  auto axis = [&](unsigned i) { return i + (i >= a ? 1u : 0u); };
+  const unsigned xf = axis(f), x1 = axis(f == 0 ? 1 : 0), x2 = axis(f == 2 ? 1 : 2);
+  const unsigned base = j * (8u >> a) + jj * (8u >> xf), w1 = 8u >> x1, w2 = 8u >> x2;
+  return uint2{base | w1 << 4 | w2 << 8 | x1 << 12 | x2 << 14 | a << 16 | xf << 18 | j << 20 | jj << 21,
+               edge_number(x1, base) | edge_number(x2, base) << 5 |
+                   edge_number(x2, base + w1) << 10 | edge_number(x1, base + w2) << 15};
+}
+__device__ __forceinline__ SquareInfo unpack_square(uint2 p) {
+  return SquareInfo{p.x & 15u,         (p.x >> 4) & 15u,  (p.x >> 8) & 15u,  (p.x >> 12) & 3u,
+                    (p.x >> 14) & 3u,  (p.x >> 16) & 3u,  (p.x >> 18) & 3u,  (p.x >> 20) & 1u,
+                    (p.x >> 21) & 1u,  p.y & 31u,         (p.y >> 5) & 31u,  (p.y >> 10) & 31u,
+                    (p.y >> 15) & 31u};
+}
+// Corners (0,0), (0,1), (1,0), (1,1) of a square above v0, as bits 0..3.
+__device__ __forceinline__ unsigned square_bits(const SquareInfo &q, unsigned m) {
+  const unsigned b = m >> q.base;
+  return (b & 1u) | ((b >> q.w2) & 1u) << 1 | ((b >> q.w1) & 1u) << 2 |
+         ((b >> (q.w1 + q.w2)) & 1u) << 3;
+}
+// First and last cut edge (0..3) of a square with two cuts.
+__device__ __forceinline__ void cut_edges(unsigned sq, unsigned &first, unsigned &last) {
+  const bool c0 = ((sq >> 2) ^ sq) & 1u, c1 = ((sq >> 1) ^ sq) & 1u;
+  const bool c2 = ((sq >> 3) ^ (sq >> 2)) & 1u, c3 = ((sq >> 3) ^ (sq >> 1)) & 1u;
+  first = c0 ? 0 : (c1 ? 1 : 2);
+  last = c3 ? 3 : (c2 ? 2 : 1);
+}
+__device__ __forceinline__ unsigned pick4(unsigned k, unsigned a, unsigned b, unsigned c,
+                                          unsigned d) {
+  return k == 0 ? a : (k == 1 ? b : (k == 2 ? c : d));
+}
+
+// LDS of a wave of plain cells; columns are lanes.  A line in the list is its
+// two edges and its square.
+template <int DIM>
+struct PlainLds {
+  static constexpr int LINES = DIM == 4 ? MAXL / 2 : 6;
+  double E[32 * 64];                     // edge cuts
+  double pc[DIM == 4 ? 8 * D * 64 : 1];  // polygon centroids, by cube
+  double2 at[32][2];                     // position of an edge: its held coordinates
+  uint2 sq[48];
+  unsigned short list[LINES * 64];       // start edge | end edge << 5 | square << 10
+};
+template <int DIM>
+__device__ __forceinline__ void plain_tables(PlainLds<DIM> &S, int lane, const double *h) {
+  if (lane < (DIM == 4 ? 48 : 6)) S.sq[lane] = pack_square(lane);
+  if (lane < 32) {
+    const unsigned d = lane >> 3, pos = lane & 7u;
+    const unsigned c = (pos >> (3 - d)) << (4 - d) | (pos & ((8u >> d) - 1u));
+    S.at[lane][0] = double2{c & 8u ? h[0] : 0.0, c & 4u ? h[1] : 0.0};
+    S.at[lane][1] = double2{c & 2u ? h[2] : 0.0, c & 1u ? h[3] : 0.0};
+  }
+}
+
+// The cut point of an edge in four coordinates.
+template <int DIM>
+__device__ __forceinline__ void edge_point(const PlainLds<DIM> &S, int lane, unsigned edge,
+                                           double *x) {
+  const double2 a = S.at[edge][0], b = S.at[edge][1];
+  const double c = S.E[64 * edge + lane];
+  const unsigned d = edge >> 3;
+  x[0] = d == 0 ? c : a.x;
+  x[1] = d == 1 ? c : a.y;
+  x[2] = d == 2 ? c : b.x;
+  x[3] = d == 3 ? c : b.y;
+}
+struct Line4 {
+  double s[D], e[D];
+};
+template <int DIM>
+__device__ __forceinline__ Line4 plain_line(const PlainLds<DIM> &S, int lane, unsigned id) {
+  Line4 l;
+  edge_point(S, lane, id & 31u, l.s);
+  edge_point(S, lane, (id >> 5) & 31u, l.e);
+  return l;
+}
+// body(line, id, whether it is a polygon's last) for the lines of the lane's
+// list; bit i of ends is set for a polygon's last line.  The next line is
+// fetched while the body works on this one: a line is two dependent LDS reads,
+// and few waves fit a CU to hide them.
+template <int DIM, typename B>
+__device__ __forceinline__ void for_lines(const PlainLds<DIM> &S, int lane, int nl,
+                                          unsigned long long ends, B &&body) {
+  unsigned id = S.list[lane];
+  Line4 l = plain_line(S, lane, id);
+#pragma unroll 1
+  for (int i = 1; i <= nl; ++i) {
+    const unsigned idn = S.list[64 * (i < nl ? i : 0) + lane];
+    const Line4 ln = plain_line(S, lane, idn);
+    body(l, id, (bool)(ends & 1ull));
+    ends >>= 1;
+    l = ln;
+    id = idn;
+  }
+}
+
+// Mean of the corners below v0 along one free axis of length h: n1 of nout
+// lie on the far side.
+__device__ __forceinline__ double outside_mean(int n1, int nout, double h) {
+  const double x = n1 == 0 ? 0.0 : (n1 == 2 ? h + h : h);
+  return nout == 1 ? x : (nout == 2 ? 0.5 * x : third(x));
+}
+// Outside point of a line (outside() of the general search).
+template <int DIM>
+__device__ __forceinline__ void plain_outside(const PlainLds<DIM> &S, unsigned id, unsigned m,
+                                              const double *h, const double *s, double *o) {
+  const SquareInfo q = unpack_square(S.sq[id >> 10]);
+  const unsigned low = ~square_bits(q, m) & 15u;
+  const int nout = __popc(low);
+  const double g0 = h[0], g1 = h[1], g2 = h[2], g3 = h[3];
+  const double h1 = q.x1 == 0 ? g0 : (q.x1 == 1 ? g1 : g2);
+  const double h2 = q.x2 == 1 ? g1 : (q.x2 == 2 ? g2 : g3);
+  const double o1 = outside_mean(__popc(low & 12u), nout, h1);
+  const double o2 = outside_mean(__popc(low & 10u), nout, h2);
+#pragma unroll
+  for (unsigned k = 0; k < D; ++k) o[k] = k == q.x1 ? o1 : (k == q.x2 ? o2 : s[k]);
+}
+
+// Lines of the hexagon of cube q in the order and direction in which the
+// general search joins them, into the list from pos on.
+template <int DIM>
+__device__ __forceinline__ void list_hexagon(PlainLds<DIM> &S, int lane, unsigned m, unsigned q,
+                                             unsigned pos) {
+  unsigned first = 0, last = 0;  // edge numbers of the six lines, five bits each
+#pragma unroll 1
+  for (unsigned r = 0; r < 6; ++r) {
+    const SquareInfo i = unpack_square(S.sq[6 * q + r]);
+    unsigned f, l;
+    cut_edges(square_bits(i, m), f, l);
+    first |= pick4(f, i.i0, i.i1, i.i2, i.i3) << (5 * r);
+    last |= pick4(l, i.i0, i.i1, i.i2, i.i3) << (5 * r);
+  }
+  unsigned end = last & 31u, free = 62u;
+  S.list[64 * pos + lane] = (unsigned short)((first & 31u) | end << 5 | (6 * q) << 10);
+#pragma unroll 1
+  for (unsigned k = 1; k < 6; ++k) {
+    unsigned next = 0, turned = 0;
+#pragma unroll
+    for (unsigned r = 5; r >= 1; --r)
+      if ((free >> r) & 1u) {
+        const bool sm = ((first >> (5 * r)) & 31u) == end, em = ((last >> (5 * r)) & 31u) == end;
+        if (sm || em) {
+          next = r;
+          turned = em ? 1u : 0u;
+        }
+      }
+    const unsigned start = ((turned ? last : first) >> (5 * next)) & 31u;
+    end = ((turned ? first : last) >> (5 * next)) & 31u;
+    free &= ~(1u << next);
+    S.list[64 * (pos + k) + lane] = (unsigned short)(start | end << 5 | (6 * q + next) << 10);
+  }
+}
+
+// Squares of the cell that are cut, and whether one is cut four times.
+template <int DIM>
+__device__ __forceinline__ unsigned long long cut_squares(unsigned m, bool &crossed) {
+  constexpr int NQ = DIM == 4 ? 8 : 1;
+  unsigned long long cut = 0;
+  crossed = false;
+#pragma unroll
+  for (unsigned q = 0; q < NQ; ++q)
+#pragma unroll
+    for (unsigned r = 0; r < 6; ++r) {
+      const unsigned a = q >> 1, f = r >> 1;
+      auto axis = [&](unsigned i) { return i + (i >= a ? 1u : 0u); };
+      const unsigned x1 = axis(f == 0 ? 1 : 0), x2 = axis(f == 2 ? 1 : 2), w1 = 8u >> x1, w2 = 8u >> x2;
+      const unsigned base = (q & 1) * (8u >> a) + (r & 1) * (8u >> axis(f));
+      const unsigned sel = (1u | 1u << w1 | 1u << w2 | 1u << (w1 + w2)) << base;
+      const unsigned in = m & sel;
+      const unsigned d1 = (1u | 1u << (w1 + w2)) << base, d2 = (1u << w1 | 1u << w2) << base;
+      if (in != 0u && in != sel) cut |= 1ull << (6 * q + r);
+      crossed = crossed || in == d1 || in == d2;
+    }
+  return cut;
+}
+
+// Lists the lines of the lane's cell (corner pattern m, edge cuts in S.E;
+// near: one of them within 1e-10 of a corner); the number of lines, or 0 if
+// the cell is not plain.  ends: the last lines of polygons.
+template <int DIM>
+__device__ __forceinline__ int list_lines(PlainLds<DIM> &S, int lane, unsigned m, bool near,
+                                          unsigned long long &ends) {
+  constexpr unsigned NQ = DIM == 4 ? 8 : 1;
+  bool crossed;
+  const unsigned long long cut = cut_squares<DIM>(m, crossed);
+  if (crossed) return 0;
+  auto lines = [&](unsigned q) { return (unsigned)(cut >> (6 * q)) & 63u; };
+  unsigned present = 0, hexagons = 0;
+#pragma unroll
+  for (unsigned q = 0; q < NQ; ++q) {
+    const unsigned f = lines(q);
+    present |= (f ? 1u : 0u) << q;
+    hexagons |= (f == 63u ? 1u : 0u) << q;
+    if (f == 63u) {
+      // two opposite corners apart from the six others: two triangles
+      const unsigned a = q >> 1, w = 8u >> a;
+      unsigned side = 0;
+#pragma unroll
+      for (unsigned c = 0; c < 16; ++c)
+        if ((c & w) == ((q & 1) ? w : 0u)) side |= 1u << c;
+      const int n = __popc(m & side);
+      if (n == 2 || n == 6) return 0;
+    }
+  }
+  const int nlines = __popcll(cut), na = __popc(m), few = na < 16 - na ? na : 16 - na;
+  bool joined = hexagons != 0u;
+  if constexpr (DIM == 4) joined = joined || (nlines == 24 && few == 2);
+  if (joined && near) return 0;
+  unsigned taken = 0, pos = 0;
+  ends = 0;
+#pragma unroll 1
+  for (unsigned t = 0; t < NQ; ++t) {
+    unsigned next = present & ~taken;
+    if (joined && taken) {
+      unsigned touch = 0;
+#pragma unroll
+      for (unsigned q = 0; q < NQ; ++q) {
+        // cubes that share a cut square with q: its squares' held axes
+        const unsigned f = lines(q), a2 = q & ~1u;
+        const unsigned adj = (f & ((1u << a2) - 1u)) | (f >> a2) << (a2 + 2);
+        touch |= (adj & taken ? 1u : 0u) << q;
+      }
+      next &= touch;
+    }
+    if (!next) break;
+    const unsigned q = (unsigned)__builtin_ctz(next);
+    taken |= 1u << q;
+    if ((hexagons >> q) & 1u) {
+      list_hexagon(S, lane, m, q, pos);
+      pos += 6;
+    } else {
+      unsigned f = (unsigned)(cut >> (6 * q)) & 63u;
+      while (f) {
+        const unsigned r = (unsigned)__builtin_ctz(f);
+        f &= f - 1u;
+        const SquareInfo i = unpack_square(S.sq[6 * q + r]);
+        unsigned a, z;
+        cut_edges(square_bits(i, m), a, z);
+        S.list[64 * pos + lane] =
+            (unsigned short)(pick4(a, i.i0, i.i1, i.i2, i.i3) |
+                             pick4(z, i.i0, i.i1, i.i2, i.i3) << 5 | (6 * q + r) << 10);
+        ++pos;
+      }
+    }
+    ends |= 1ull << (pos - 1);
+  }
+  return taken == present ? (int)pos : 0;
+}
+
+// Element of the lane's plain 4-D cell of nl lines.  The sums are those of
+// polygon_geometry and polyhedron_geometry, term by term.
+__device__ __forceinline__ void plain_element4(PlainLds<4> &S, int lane, unsigned m, int nl,
+                                               unsigned long long ends, const double *h, double *cen,
+                                               double *nrm) {
+  auto pc = [&](unsigned id, int k) -> double & { return S.pc[64 * ((id >> 10) / 6 * D + k) + lane]; };
+  // polygon means and the mean of all lines
+  double mean[D] = {0, 0, 0, 0}, pm[D] = {0, 0, 0, 0};
+  int n = 0;
+  for_lines(S, lane, nl, ends, [&](const Line4 &l, unsigned id, bool last) {
+    for (int k = 0; k < D; ++k) {
+      const double t = l.s[k] + l.e[k];
+      pm[k] += t;
+      mean[k] += t;
+    }
+    ++n;
+    if (last) {
+      for (int k = 0; k < D; ++k) {
+        pc(id, k) = pm[k] / double(2.0 * n);
+        pm[k] = 0;
+      }
+      n = 0;
+    }
+  });
+  for (int k = 0; k < D; ++k) mean[k] = mean[k] / double(2.0 * nl);
+  // area-weighted centroids of the polygons with more than three lines
+  double up[D] = {0, 0, 0, 0}, down = 0;
+  for_lines(S, lane, nl, ends, [&](const Line4 &l, unsigned id, bool last) {
+    double a[D], b[D], c[D];
+    for (int k = 0; k < D; ++k) {
+      c[k] = pc(id, k);
+      a[k] = l.s[k] - c[k];
+      b[k] = l.e[k] - c[k];
+    }
+    // the cube's free axes in order
+    const unsigned held = (id >> 10) / 12;
+    auto free_axis = [&](const double *v, int i) {
+      return (unsigned)i < held ? v[i] : v[i + 1];
+    };
+    const double a1 = free_axis(a, 0), a2 = free_axis(a, 1), a3 = free_axis(a, 2);
+    const double b1 = free_axis(b, 0), b2 = free_axis(b, 1), b3 = free_axis(b, 2);
+    const double u1 = a2 * b3 - a3 * b2;
+    const double u2 = a1 * b3 - a3 * b1;
+    const double u3 = a2 * b1 - a1 * b2;
+    const double ar = 0.5 * sqrt(u1 * u1 + u2 * u2 + u3 * u3);
+    for (int k = 0; k < D; ++k) up[k] += third(l.s[k] + l.e[k] + c[k]) * ar;
+    down += ar;
+    ++n;
+    if (last) {
+      if (n > 3)
+        for (int k = 0; k < D; ++k) pc(id, k) = up[k] / down;
+      for (int k = 0; k < D; ++k) up[k] = 0;
+      down = 0;
+      n = 0;
+    }
+  });
+  // volume-weighted centroid of the polyhedron
+  for_lines(S, lane, nl, ends, [&](const Line4 &l, unsigned id, bool) {
+    double a[D], b[D], c[D], t[D];
+    for (int k = 0; k < D; ++k) {
+      t[k] = pc(id, k);
+      a[k] = l.s[k] - mean[k];
+      b[k] = l.e[k] - mean[k];
+      c[k] = t[k] - mean[k];
+      t[k] = (l.s[k] + l.e[k] + t[k] + mean[k]) / 4.0;
+    }
+    double nv[D];
+    tetra_normal(a, b, c, nv);
+    double V = 0;
+    for (int k = 0; k < D; ++k) V += nv[k] * nv[k];
+    V = sqrt(V);
+    for (int k = 0; k < D; ++k) up[k] += t[k] * V;
+    down += V;
+  });
+  for (int k = 0; k < D; ++k) cen[k] = up[k] / down;
+  // oriented normal
+  for (int k = 0; k < D; ++k) nrm[k] = 0;
+  for_lines(S, lane, nl, ends, [&](const Line4 &l, unsigned id, bool) {
+    double a[D], b[D], c[D], o[D], nv[D];
+    plain_outside(S, id, m, h, l.s, o);
+    for (int k = 0; k < D; ++k) {
+      a[k] = l.s[k] - cen[k];
+      b[k] = l.e[k] - cen[k];
+      c[k] = pc(id, k) - cen[k];
+      o[k] = o[k] - cen[k];
+    }
+    tetra_normal(a, b, c, nv);
+    orient(nv, o);
+    for (int k = 0; k < D; ++k) nrm[k] += nv[k];
+  });
+}
+
+// The same for a plain 3-D cell, the cube with axis 0 held at 0.
+__device__ __forceinline__ void plain_element3(PlainLds<3> &S, int lane, unsigned m, int nl,
+                                               const double *h, double *cen, double *nrm) {
+  double pm[D] = {0, 0, 0, 0};
+  for_lines(S, lane, nl, 0, [&](const Line4 &l, unsigned, bool) {
+    for (int k = 0; k < D; ++k) pm[k] += l.s[k] + l.e[k];
+  });
+  for (int k = 0; k < D; ++k) pm[k] = pm[k] / double(2.0 * nl);
+  if (nl > 3) {
+    double up[D] = {0, 0, 0, 0}, down = 0;
+    for_lines(S, lane, nl, 0, [&](const Line4 &l, unsigned, bool) {
+      double a[D], b[D];
+      for (int k = 0; k < D; ++k) {
+        a[k] = l.s[k] - pm[k];
+        b[k] = l.e[k] - pm[k];
+      }
+      const double u1 = a[2] * b[3] - a[3] * b[2];
+      const double u2 = a[1] * b[3] - a[3] * b[1];
+      const double u3 = a[2] * b[1] - a[1] * b[2];
+      const double ar = 0.5 * sqrt(u1 * u1 + u2 * u2 + u3 * u3);
+      for (int k = 0; k < D; ++k) up[k] += third(l.s[k] + l.e[k] + pm[k]) * ar;
+      down += ar;
+    });
+    for (int k = 0; k < D; ++k) pm[k] = up[k] / down;
+  }
+  for (int k = 0; k < D; ++k) {
+    cen[k] = pm[k];
+    nrm[k] = 0;
+  }
+  for_lines(S, lane, nl, 0, [&](const Line4 &l, unsigned id, bool) {
+    double a[D], b[D], o[D], t[D];
+    plain_outside(S, id, m, h, l.s, o);
+    for (int k = 0; k < D; ++k) {
+      a[k] = l.s[k] - pm[k];
+      b[k] = l.e[k] - pm[k];
+      o[k] = o[k] - pm[k];
+    }
+    t[0] = 0.0;
+    t[1] = 0.5 * (a[2] * b[3] - a[3] * b[2]);
+    t[2] = -0.5 * (a[1] * b[3] - a[3] * b[1]);
+    t[3] = 0.5 * (a[1] * b[2] - a[2] * b[1]);
+    orient(t, o);
+    for (int k = 0; k < D; ++k) nrm[k] += t[k];
+  });
+}
+
 }  // namespace corn
 }  // namespace gvh

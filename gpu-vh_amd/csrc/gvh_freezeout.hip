@@ -14,8 +14,10 @@
 //     the window walks eta, so neighbouring threads read neighbouring cells;
 //     counts per row, an exclusive scan and a second walk give the surface
 //     cubes in the reference's (it, ix, iy, ieta) order.
-//  3. fo_cornelius_kernel: one wave per surface cube, elements via the LDS
-//     restatement of cornelius (gvh_cornelius.h).
+//  3. fo_plain_cells_kernel: one lane per surface cube whose lines need no
+//     joining, which is nearly all of them; fo_cornelius_kernel: one wave per
+//     cube for the rest, via the LDS restatement of cornelius
+//     (gvh_cornelius.h).
 //  4. fo_emit_kernel: one thread per (element, variable) writes the rows
 //     (position, normal, multilinearly interpolated hydro variables, T and P
 //     of the interpolated e), offsets from a scan of element counts.
@@ -72,7 +74,8 @@ struct FoState {
   // window buffers, grown on demand
   unsigned *rowcnt = nullptr, *rowoff = nullptr;
   size_t row_cap = 0;           // rowcnt and rowoff
-  unsigned *cubes = nullptr;     // cubes, ecnt, eoff, elem: cube_cap
+  unsigned *cubes = nullptr;     // cubes, rest, ecnt, eoff, elem: cube_cap
+  unsigned *rest = nullptr;      // cubes left to the general search
   int *ecnt = nullptr;
   unsigned *eoff = nullptr;
   double *elem = nullptr;
@@ -81,10 +84,10 @@ struct FoState {
   size_t rows_cap = 0;
   unsigned *scan_tmp = nullptr;
   size_t scan_cap = 0;
-  unsigned *total = nullptr;  // device scalars: [0] scan total, [1] overflow
+  unsigned *total = nullptr;  // device scalars: [0] scan total, [2] overflow, [3] size of rest
   long long ncubes = 0, nrows = 0;
   // the window search in progress (fo_find_count .. fo_find_emit)
-  unsigned htot[2] = {0, 0};  // host copies of total[0], total[1]
+  unsigned htot[4] = {0, 0, 0, 0};  // host copy of total
   long long nrow_pending = 0;
   int n_pending = 0;
 };
@@ -93,7 +96,7 @@ double *fo_ring(FoState *f) { return f ? f->ring : nullptr; }
 
 void fo_free(FoState *f) {
   if (!f) return;
-  for (void *p : {(void *)f->ring, (void *)f->rowcnt, (void *)f->rowoff, (void *)f->cubes,
+  for (void *p : {(void *)f->ring, (void *)f->rowcnt, (void *)f->rowoff, (void *)f->cubes, (void *)f->rest,
                   (void *)f->ecnt, (void *)f->eoff, (void *)f->elem, (void *)f->rows,
                   (void *)f->scan_tmp, (void *)f->total})
     if (p) (void)hipFree(p);
@@ -305,53 +308,115 @@ struct CellSource {
   bool window;
 };
 
-__global__ __launch_bounds__(64) void fo_cornelius_kernel(CellSource S, long long ncells, int dim,
-                                                          double dx0, double dx1, double dx2,
-                                                          double dx3, double v0,
+// Corner `c` of cell `cell` (index over (it, ix, iy[, iz]), last axis fastest).
+template <int DIM>
+__device__ __forceinline__ double cell_corner(const CellSource &S, long long cell, int c, int itl,
+                                              int ix, int iy, int iz) {
+  if (!S.window) return S.corners[cell * (1 << DIM) + c];
+  const int a = c >> (DIM - 1), b = (c >> (DIM - 2)) & 1, y = (c >> (DIM - 3)) & 1;
+  const int z = DIM == 4 ? c & 1 : 0;
+  return S.W.e_slot(S.W.start + itl + a)[S.W.cell(ix + b, iy + y, iz + z)];
+}
+
+struct Spacing {
+  double dx[4];  // of the 4-vectors: dx[0] is 1 in 3-D
+  double v0;
+};
+
+// Plain cells, one per lane (gvh_cornelius.h): their elements, and the list
+// of the other surface cells for the general search.  What bounds it is
+// latency: four walks over some 28 lines, each two dependent LDS reads, and
+// the edge cuts and polygon centroids of 64 cells (40 KB in 4-D) leave one
+// wave per SIMD.  206 448 surface cubes of a 121x121x61 window: 326 us with the
+// general search of the rest, against 1590 us with a wave per cube for all;
+// 850 000 of a 201x201x101 window 1.07 against 6.14 ms.
+template <int DIM>
+__global__ __launch_bounds__(64) void fo_plain_cells_kernel(CellSource S, long long ncells,
+                                                            Spacing sp, int *__restrict__ ecnt,
+                                                            double *__restrict__ elem,
+                                                            unsigned *__restrict__ rest,
+                                                            unsigned *__restrict__ nrest) {
+  constexpr int NC = 1 << DIM;
+  __shared__ corn::PlainLds<DIM> L;
+  const int lane = threadIdx.x;
+  const long long cell = (long long)blockIdx.x * 64 + lane;
+  corn::plain_tables(L, lane, sp.dx);
+  __syncthreads();
+  bool general = false;
+  int nl = 0;
+  unsigned m = 0;
+  unsigned long long ends = 0;
+  if (cell < ncells) {
+    int itl = 0, ix = 0, iy = 0, iz = 0;
+    if (S.window) decode_cube(S.W, S.cubes[cell], itl, ix, iy, iz);
+    double v[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) v[c] = cell_corner<DIM>(S, cell, c, itl, ix, iy, iz);
+    const bool ok = corn::corner_mask<NC>(v, sp.v0, m);
+    const bool surface = m != 0u && m != (1u << NC) - 1u;
+    if (surface && ok) {
+      bool near = false;
+#pragma unroll
+      for (int d = 4 - DIM; d < 4; ++d)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          const int w = 8 >> d;
+          if (c & w) continue;
+          if (((m >> c) ^ (m >> (c + w))) & 1u) {
+            const double x = corn::edge_cut(v[c], v[c + w], sp.v0, sp.dx[d]);
+            near = near || !(x > 2e-10 && sp.dx[d] - x > 2e-10);
+            L.E[64 * corn::edge_number(d, c) + lane] = x;
+          }
+        }
+      nl = corn::list_lines(L, lane, m, near, ends);
+    }
+    general = surface && nl == 0;
+    if (!general) ecnt[cell] = surface ? 1 : 0;
+  }
+  // the others, in any order: one atomic per wave
+  const unsigned long long g = __ballot(general);
+  if (g) {
+    unsigned base = 0;
+    if (lane == 0) base = atomicAdd(nrest, (unsigned)__popcll(g));
+    base = __shfl(base, 0, 64);
+    if (general) rest[base + __popcll(g & ((1ull << lane) - 1ull))] = (unsigned)cell;
+  }
+  if (nl == 0) return;
+  double cen[4], nrm[4];
+  if constexpr (DIM == 4) corn::plain_element4(L, lane, m, nl, ends, sp.dx, cen, nrm);
+  else corn::plain_element3(L, lane, m, nl, sp.dx, cen, nrm);
+  double *o = elem + cell * corn::MAXE * ELEM;
+  for (int k = 0; k < 4; ++k) {
+    o[k] = cen[k];
+    o[4 + k] = nrm[k];
+  }
+}
+
+// The general search of the listed cells, one wave per cell.
+template <int DIM>
+__global__ __launch_bounds__(64) void fo_cornelius_kernel(CellSource S, Spacing sp,
+                                                          const unsigned *__restrict__ rest,
+                                                          const unsigned *__restrict__ nrest,
                                                           int *__restrict__ ecnt,
                                                           double *__restrict__ elem,
                                                           unsigned *__restrict__ overflow) {
   __shared__ corn::Work W;
   __shared__ double cen[corn::MAXE][corn::D], nrm[corn::MAXE][corn::D];
   const int lane = threadIdx.x;
-  const int ncorner = 1 << dim;
-  // one block (wave) per cell: cells differ much in cost, and the dispatcher
-  // balances single-cell blocks better than a loop over a fixed grid
-  {
-    const long long cell = blockIdx.x;
-    if (cell >= ncells) return;
+  const unsigned n_rest = *nrest;
+#pragma unroll 1
+  for (unsigned r = blockIdx.x; r < n_rest; r += gridDim.x) {
+    const long long cell = rest[r];
     if (lane == 0) {
-      W.dim = dim;
-      W.v0 = v0;
-      W.dx[0] = dim == 4 ? dx0 : 1.0;
-      W.dx[1] = dim == 4 ? dx1 : dx0;
-      W.dx[2] = dim == 4 ? dx2 : dx1;
-      W.dx[3] = dim == 4 ? dx3 : dx2;
+      W.dim = DIM;
+      W.v0 = sp.v0;
+      for (int k = 0; k < 4; ++k) W.dx[k] = sp.dx[k];
       W.overflow = 0;
     }
-    if (lane < ncorner) {
-      double v;
-      if (S.window) {
-        int itl, ix, iy, iz;
-        decode_cube(S.W, S.cubes[cell], itl, ix, iy, iz);
-        // corner index over (it, ix, iy[, iz]), last axis fastest
-        int a, b, c, d;
-        if (dim == 4) {
-          a = lane >> 3;
-          b = (lane >> 2) & 1;
-          c = (lane >> 1) & 1;
-          d = lane & 1;
-        } else {
-          a = lane >> 2;
-          b = (lane >> 1) & 1;
-          c = lane & 1;
-          d = 0;
-        }
-        v = S.W.e_slot(S.W.start + itl + a)[S.W.cell(ix + b, iy + c, iz + d)];
-      } else {
-        v = S.corners[cell * ncorner + lane];
-      }
-      W.v[lane] = v;
+    if (lane < 1 << DIM) {
+      int itl = 0, ix = 0, iy = 0, iz = 0;
+      if (S.window) decode_cube(S.W, S.cubes[cell], itl, ix, iy, iz);
+      W.v[lane] = cell_corner<DIM>(S, cell, lane, itl, ix, iy, iz);
     }
     __syncthreads();
     const int n = corn::cell_elements(W, cen, nrm);
@@ -367,6 +432,33 @@ __global__ __launch_bounds__(64) void fo_cornelius_kernel(CellSource S, long lon
     }
     __syncthreads();
   }
+}
+
+// Elements of ncells cells into ecnt and elem.  counts: two 32-bit words, the
+// cells with more than MAXE elements and those left to the general search;
+// rest: room for ncells numbers.
+template <int DIM>
+hipError_t launch_cornelius_d(const CellSource &S, long long ncells, const Spacing &sp, int *ecnt,
+                              double *elem, unsigned *counts, unsigned *rest, hipStream_t st) {
+  hipError_t e = launch_fill_u64(reinterpret_cast<unsigned long long *>(counts), 1, 0ull, st);
+  if (e != hipSuccess) return e;
+  fo_plain_cells_kernel<DIM><<<(unsigned)((ncells + 63) / 64), 64, 0, st>>>(S, ncells, sp, ecnt, elem,
+                                                                          rest, counts + 1);
+  e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  // ten waves fit a CU's LDS
+  const unsigned grid = (unsigned)std::min<long long>(ncells, 2560);
+  fo_cornelius_kernel<DIM><<<grid, 64, 0, st>>>(S, sp, rest, counts + 1, ecnt, elem, counts);
+  return hipGetLastError();
+}
+hipError_t launch_cornelius(const CellSource &S, long long ncells, int dim, double dx0, double dx1,
+                            double dx2, double dx3, double v0, int *ecnt, double *elem,
+                            unsigned *counts, unsigned *rest, hipStream_t st) {
+  if (dim == 4)
+    return launch_cornelius_d<4>(S, ncells, Spacing{{dx0, dx1, dx2, dx3}, v0}, ecnt, elem, counts,
+                                 rest, st);
+  return launch_cornelius_d<3>(S, ncells, Spacing{{1.0, dx0, dx1, dx2}, v0}, ecnt, elem, counts,
+                               rest, st);
 }
 
 // ------------------------------------------------------------------ emit
@@ -542,7 +634,8 @@ int ensure_cubes(FoState *f, size_t ncubes) {
   if (ncubes <= f->cube_cap) return GVH_OK;
   const size_t cap = with_headroom(ncubes);
   int rc;
-  if ((rc = realloc_dev(f->cubes, cap, 1)) || (rc = realloc_dev(f->ecnt, cap, 1)) ||
+  if ((rc = realloc_dev(f->cubes, cap, 1)) || (rc = realloc_dev(f->rest, cap, 1)) ||
+      (rc = realloc_dev(f->ecnt, cap, 1)) ||
       (rc = realloc_dev(f->eoff, cap, 1)) ||
       (rc = realloc_dev(f->elem, cap, (size_t)corn::MAXE * ELEM))) {
     f->cube_cap = 0;
@@ -629,7 +722,7 @@ int fo_init(gvh_context *c, int fofreq, double e_fo, int flags, int halves) {
   const size_t bytes = (size_t)halves * (fofreq + 1) * NVAR * nint * sizeof(double);
   hipError_t e = hipMalloc((void **)&f->ring, bytes);
   if (e == hipSuccess) e = hipMemsetAsync(f->ring, 0, bytes, c->stream);
-  if (e == hipSuccess) e = hipMalloc((void **)&f->total, 2 * sizeof(unsigned));
+  if (e == hipSuccess) e = hipMalloc((void **)&f->total, 4 * sizeof(unsigned));
   if (e != hipSuccess) {
     fo_free(f);
     return gvh_fail(GVH_ENOMEM, "freeze-out history of %zu bytes: %s", bytes, hipGetErrorString(e));
@@ -715,7 +808,7 @@ int fo_find_elements(gvh_context *c, hipStream_t st) {
   const long long ncubes = f->htot[0];
   f->ncubes = ncubes;
   if (ncubes == 0) {
-    f->htot[0] = f->htot[1] = 0;
+    f->htot[0] = f->htot[2] = 0;
     return GVH_OK;
   }
   const int start = f->n_pending <= f->fofreq ? 2 : 0;
@@ -726,22 +819,15 @@ int fo_find_elements(gvh_context *c, hipStream_t st) {
                                                                         f->cubes);
   HIP_TRY(hipGetLastError());
   CellSource S{W, f->cubes, nullptr, true};
-  HIP_TRY(hipMemsetAsync(f->total + 1, 0, sizeof(unsigned), st));
   if (ncubes > 0x7fffffffLL) return gvh_fail(GVH_EINVAL, "%lld surface cubes in one window", ncubes);
-  const unsigned grid = (unsigned)ncubes;
   const double dz = c->L.latticeSpacingRapidity;
   const double dt = c->L.latticeSpacingProperTime, dx = c->L.latticeSpacingX,
                dy = c->L.latticeSpacingY;
-  if (f->dim == 4)
-    fo_cornelius_kernel<<<grid, 64, 0, st>>>(S, ncubes, 4, dt, dx, dy, dz, f->e_fo, f->ecnt,
-                                             f->elem, f->total + 1);
-  else
-    fo_cornelius_kernel<<<grid, 64, 0, st>>>(S, ncubes, 3, dt, dx, dy, 0.0, f->e_fo, f->ecnt,
-                                             f->elem, f->total + 1);
-  HIP_TRY(hipGetLastError());
+  HIP_TRY(launch_cornelius(S, ncubes, f->dim, dt, dx, dy, dz, f->e_fo, f->ecnt, f->elem,
+                           f->total + 2, f->rest, st));
   HIP_TRY(scan_with_total((const unsigned *)f->ecnt, f->eoff, (size_t)ncubes, f->scan_tmp,
                           f->total, st));
-  HIP_TRY(hipMemcpyAsync(f->htot, f->total, 2 * sizeof(unsigned), hipMemcpyDeviceToHost, st));
+  HIP_TRY(hipMemcpyAsync(f->htot, f->total, 4 * sizeof(unsigned), hipMemcpyDeviceToHost, st));
   return GVH_OK;
 }
 
@@ -751,8 +837,8 @@ int fo_find_emit(gvh_context *c, double t, hipStream_t st, long long *nelements)
   FoState *f = c->fo;
   *nelements = 0;
   if (f->ncubes == 0) return GVH_OK;
-  if (f->htot[1])
-    return gvh_fail(GVH_EINVAL, "%u freeze-out cells exceed %d elements", f->htot[1], corn::MAXE);
+  if (f->htot[2])
+    return gvh_fail(GVH_EINVAL, "%u freeze-out cells exceed %d elements", f->htot[2], corn::MAXE);
   const long long nrows = f->htot[0];
   int rc;
   if ((rc = ensure_out_rows(f, (size_t)nrows))) return rc;
@@ -847,21 +933,19 @@ extern "C" int gvh_cornelius_cells(int dim, long long ncells, const double *corn
   const int ncorner = 1 << dim;
   double *dv = nullptr, *del = nullptr;
   int *dcnt = nullptr;
-  unsigned *dov = nullptr;
+  unsigned *dov = nullptr, *drest = nullptr;
   hipError_t e = hipMalloc((void **)&dv, (size_t)ncells * ncorner * sizeof(double));
   if (e == hipSuccess) e = hipMalloc((void **)&del, (size_t)ncells * corn::MAXE * ELEM * sizeof(double));
   if (e == hipSuccess) e = hipMalloc((void **)&dcnt, (size_t)ncells * sizeof(int));
-  if (e == hipSuccess) e = hipMalloc((void **)&dov, sizeof(unsigned));
+  if (e == hipSuccess) e = hipMalloc((void **)&dov, 2 * sizeof(unsigned));
+  if (e == hipSuccess) e = hipMalloc((void **)&drest, (size_t)ncells * sizeof(unsigned));
   if (e == hipSuccess) e = hipMemcpy(dv, corners, (size_t)ncells * ncorner * sizeof(double), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemset(dov, 0, sizeof(unsigned));
   if (e == hipSuccess) {
     CellSource S{};
     S.window = false;
     S.corners = dv;
-    const unsigned grid = (unsigned)ncells;
-    fo_cornelius_kernel<<<grid, 64>>>(S, ncells, dim, dx[0], dx[1], dx[2], dim == 4 ? dx[3] : 0.0,
-                                      v0, dcnt, del, dov);
-    e = hipGetLastError();
+    e = launch_cornelius(S, ncells, dim, dx[0], dx[1], dx[2], dim == 4 ? dx[3] : 0.0, v0, dcnt, del,
+                         dov, drest, nullptr);
   }
   std::vector<double> el;
   unsigned ov = 0;
@@ -871,7 +955,7 @@ extern "C" int gvh_cornelius_cells(int dim, long long ncells, const double *corn
   }
   if (e == hipSuccess) e = hipMemcpy(counts, dcnt, (size_t)ncells * sizeof(int), hipMemcpyDeviceToHost);
   if (e == hipSuccess) e = hipMemcpy(&ov, dov, sizeof ov, hipMemcpyDeviceToHost);
-  for (void *p : {(void *)dv, (void *)del, (void *)dcnt, (void *)dov})
+  for (void *p : {(void *)dv, (void *)del, (void *)dcnt, (void *)dov, (void *)drest})
     if (p) (void)hipFree(p);
   if (e != hipSuccess) return gvh_fail(GVH_EHIP, "gvh_cornelius_cells: %s", hipGetErrorString(e));
   const int off = dim == 4 ? 0 : 1;
@@ -896,9 +980,9 @@ namespace {
 
 constexpr long long NA_MAX_CELLS = GVH_CORNELIUS_NOALLOC_MAX_CELLS;
 constexpr long long NA_ELEM_DOUBLES = NA_MAX_CELLS * corn::MAXE * ELEM;
-// element records, then one 64-bit word holding the overflow counter (the
-// tail is padded to 256 bytes)
-static __device__ __align__(256) double scratch[NA_ELEM_DOUBLES + 32];
+// element records, then one 64-bit word holding the two counters of
+// launch_cornelius (padded to 256 bytes), then its list of cells
+static __device__ __align__(256) double scratch[NA_ELEM_DOUBLES + 32 + NA_MAX_CELLS / 2];
 
 constexpr int NA_MAX_DEVICES = 64;
 std::mutex na_mutex;
@@ -961,22 +1045,19 @@ extern "C" int gvh_cornelius_cells_noalloc(int dim, long long ncells, const doub
   double *elem = base;
   unsigned long long *ov_word = reinterpret_cast<unsigned long long *>(base + NA_ELEM_DOUBLES);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // the counter keeps the last call's value: clear it in the stream
-  HIP_TRY(launch_fill_u64(ov_word, 1, 0ull, st));
   CellSource S{};
   S.window = false;
   S.corners = corners;
-  hipLaunchKernelGGL(fo_cornelius_kernel, dim3((unsigned)ncells), dim3(64), 0, st, S, ncells, dim,
-                     dx[0], dx[1], dx[2], dim == 4 ? dx[3] : 0.0, v0, counts, elem,
-                     reinterpret_cast<unsigned *>(ov_word));
-  HIP_TRY(hipGetLastError());
+  HIP_TRY(launch_cornelius(S, ncells, dim, dx[0], dx[1], dx[2], dim == 4 ? dx[3] : 0.0, v0, counts,
+                           elem, reinterpret_cast<unsigned *>(ov_word),
+                           reinterpret_cast<unsigned *>(base + NA_ELEM_DOUBLES + 32), st));
   const long long nslots = ncells * corn::MAXE;
   hipLaunchKernelGGL(cornelius_unpack_kernel, dim3((unsigned)((nslots + 255) / 256)), dim3(256), 0,
                      st, ncells, dim, counts, elem, centroids, normals);
   HIP_TRY(hipGetLastError());
-  unsigned long long ov = 0;
+  unsigned ov = 0;
   HIP_TRY(hipMemcpyAsync(&ov, ov_word, sizeof ov, hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
-  if (ov) return gvh_fail(GVH_EINVAL, "%llu cells exceed %d elements", ov, corn::MAXE);
+  if (ov) return gvh_fail(GVH_EINVAL, "%u cells exceed %d elements", ov, corn::MAXE);
   return GVH_OK;
 }
