@@ -20,6 +20,7 @@
 #include "../../include/gpuvh.h"
 #include "gvh_device.h"
 #include "gvh_internal.h"
+#include "gvh_state.h"
 
 namespace gvh {
 hipError_t launch_stage(const StageArgs &A, int eos, bool bulk, bool stage2, int precision,
@@ -357,27 +358,12 @@ extern "C" int gvh_destroy(gvh_context *c) {
   return GVH_OK;
 }
 
-// ghost fill on the host copy of the initial state (GhostCells.cu:66-144)
-static void host_ghosts(std::vector<double *> &arrs, int nx, int ny, int nz, int ncx, int ncy) {
-  auto id = [&](int i, int j, int k) { return (size_t)i + (size_t)ncx * (j + (size_t)ncy * k); };
-  for (double *a : arrs) {
-    for (int k = 2; k < nz + 2; ++k)
-      for (int j = 2; j < ny + 2; ++j) {
-        a[id(0, j, k)] = a[id(1, j, k)] = a[id(2, j, k)];
-        a[id(nx + 2, j, k)] = a[id(nx + 3, j, k)] = a[id(nx + 1, j, k)];
-      }
-    for (int k = 2; k < nz + 2; ++k)
-      for (int i = 2; i < nx + 2; ++i) {
-        a[id(i, 0, k)] = a[id(i, 1, k)] = a[id(i, 2, k)];
-        a[id(i, ny + 2, k)] = a[id(i, ny + 3, k)] = a[id(i, ny + 1, k)];
-      }
-    for (int j = 2; j < ny + 2; ++j)
-      for (int i = 2; i < nx + 2; ++i) {
-        a[id(i, j, 0)] = a[id(i, j, 1)] = a[id(i, j, 2)];
-        a[id(i, j, nz + 2)] = a[id(i, j, nz + 3)] = a[id(i, j, nz + 1)];
-      }
-  }
-}
+static Extent extent_of(const gvh_context *c) { return Extent{c->G, c->nx, c->ny, c->nz, c->ncx, c->ncy}; }
+
+// Transfers pass through the predictor's buffer, whose contents a step does
+// not outlive: qstride doubles (at least 9.5 G), in stream order with the
+// steps.
+static double *transfer_scratch(gvh_context *c) { return c->qbuf[2]; }
 
 extern "C" int gvh_set_initial_state(gvh_context *c, double t0, const double *e, const double *p,
                                      const double *ut, const double *ux, const double *uy,
@@ -385,58 +371,42 @@ extern "C" int gvh_set_initial_state(gvh_context *c, double t0, const double *e,
   (void)t0;
   if (!c || !e || !p || !ut || !ux || !uy || !un)
     return gvh_fail(GVH_EINVAL, "gvh_set_initial_state: NULL argument");
-  const int nx = c->nx, ny = c->ny, nz = c->nz, ncx = c->ncx, ncy = c->ncy;
-  const size_t G = (size_t)c->G, nint = (size_t)nx * ny * nz;
-  // host image of one conserved buffer, e, p and u (zero outside the interior)
-  std::vector<double> hq(15 * G, 0.0), he(G, 0.0), hp(G, 0.0), hu(4 * G, 0.0), hup(4 * G, 0.0);
-  for (int k = 0; k < nz; ++k)
-    for (int j = 0; j < ny; ++j)
-      for (int i = 0; i < nx; ++i) {
-        const size_t a = i + (size_t)nx * (j + (size_t)ny * k);
-        const size_t s = (i + 2) + (size_t)ncx * ((j + 2) + (size_t)ncy * (k + 2));
-        const double Pis = (Pi && c->bulk) ? Pi[a] : 0.0;
-        he[s] = e[a];
-        hp[s] = p[a];
-        hu[s] = ut[a];
-        hu[G + s] = ux[a];
-        hu[2 * G + s] = uy[a];
-        hu[3 * G + s] = un[a];
-        for (int m = 0; m < 10; ++m) hq[(4 + m) * G + s] = pi10 ? pi10[m * nint + a] : 0.0;
-        if (c->bulk) hq[14 * G + s] = Pis;
-        // setConservedVariables with Ttt..Ttn (EnergyMomentumTensor.cu:159-177)
-        const double P = p[a] + Pis;
-        hq[0 * G + s] = (e[a] + P) * ut[a] * ut[a] - P + hq[4 * G + s];
-        hq[1 * G + s] = (e[a] + P) * ut[a] * ux[a] + hq[5 * G + s];
-        hq[2 * G + s] = (e[a] + P) * ut[a] * uy[a] + hq[6 * G + s];
-        hq[3 * G + s] = (e[a] + P) * ut[a] * un[a] + hq[7 * G + s];
-      }
-  hup = hu;  // the previous-step velocity has zero ghosts (DynamicalVariables.cu:280-284)
-  std::vector<double *> arrs;
-  for (int n = 0; n < 15; ++n) arrs.push_back(hq.data() + n * G);
-  arrs.push_back(he.data());
-  arrs.push_back(hp.data());
-  for (int m = 0; m < 4; ++m) arrs.push_back(hu.data() + m * G);
-  host_ghosts(arrs, nx, ny, nz, ncx, ncy);
-
+  const size_t nint = (size_t)c->nx * c->ny * c->nz;
   c->iq = 0;
   c->iu = 0;
   c->iup = 1;
   c->ie = 0;
-  const size_t B = sizeof(double);
-  std::vector<float> hqf;
-  if (c->precision != GVH_FP64) {
-    // T^{tau mu} in FP64, pi and Pi stored in FP32
-    hqf.assign(hq.begin() + 4 * G, hq.end());
-    HIP_TRY(hipMemcpyAsync(c->qbuf[c->iq], hq.data(), 4 * G * B, hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(hipMemcpyAsync(c->qbuf[c->iq] + 4 * G, hqf.data(), 11 * G * sizeof(float),
-                           hipMemcpyHostToDevice, c->stream));
-  } else {
-    HIP_TRY(hipMemcpyAsync(c->qbuf[c->iq], hq.data(), 15 * G * B, hipMemcpyHostToDevice, c->stream));
-  }
-  HIP_TRY(hipMemcpyAsync(c->ebuf[c->ie], he.data(), G * B, hipMemcpyHostToDevice, c->stream));
-  HIP_TRY(hipMemcpyAsync(c->pbuf[c->ie], hp.data(), G * B, hipMemcpyHostToDevice, c->stream));
-  HIP_TRY(hipMemcpyAsync(c->ubuf[c->iu], hu.data(), 4 * G * B, hipMemcpyHostToDevice, c->stream));
-  HIP_TRY(hipMemcpyAsync(c->ubuf[c->iup], hup.data(), 4 * G * B, hipMemcpyHostToDevice, c->stream));
+  // Eleven fields at most are on the device at a time: nine of them in the
+  // scratch (9 G fit) and two in the stage's e and p buffers.
+  double *dev[11];
+  for (int m = 0; m < 9; ++m) dev[m] = transfer_scratch(c) + (size_t)m * c->G;
+  dev[9] = c->ebuf[1];
+  dev[10] = c->pbuf[1];
+  int used = 0;
+  auto upload = [&](const double *host, const double *&field) -> int {
+    field = nullptr;
+    if (!host) return GVH_OK;
+    HIP_TRY(hipMemcpyAsync(dev[used], host, nint * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    field = dev[used++];
+    return GVH_OK;
+  };
+  const StateBlocks B{c->qbuf[c->iq], c->ebuf[c->ie], c->pbuf[c->ie], c->ubuf[c->iu], c->ubuf[c->iup]};
+  const Extent X = extent_of(c);
+  const bool mixed = c->precision != GVH_FP64;
+  InitialFields F{};
+  int rc;
+  const double *u[4] = {ut, ux, uy, un};
+  if ((rc = upload(e, F.e)) || (rc = upload(p, F.p))) return rc;
+  for (int m = 0; m < 4; ++m)
+    if ((rc = upload(u[m], F.u[m]))) return rc;
+  for (int m = 0; m < 4; ++m)
+    if ((rc = upload(pi10 ? pi10 + m * nint : nullptr, F.pi[m]))) return rc;
+  if ((rc = upload(c->bulk ? Pi : nullptr, F.Pi))) return rc;
+  HIP_TRY(launch_state(F, B, X, mixed, false, c->stream));
+  used = 0;
+  for (int m = 4; m < 10; ++m)
+    if ((rc = upload(pi10 ? pi10 + m * nint : nullptr, F.pi[m]))) return rc;
+  HIP_TRY(launch_state(F, B, X, mixed, true, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
   c->initialized = true;
   c->steps_done = 0;
@@ -462,19 +432,27 @@ static void *field_dev(gvh_context *c, int f, bool *is_float) {
   return nullptr;
 }
 
-int gvh_copy_q_field(gvh_context *c, const double *qbase, int f, double *host) {
-  const size_t G = (size_t)c->G;
-  if (c->precision != GVH_FP64 && f >= GVH_PITT) {
-    std::vector<float> tmp(G);
-    HIP_TRY(hipMemcpyAsync(tmp.data(), reinterpret_cast<const float *>(qbase + 4 * G) + (f - GVH_PITT) * G,
-                           G * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    for (size_t i = 0; i < G; ++i) host[i] = tmp[i];
-    return GVH_OK;
+// A ghosted block to the host as doubles, packed on the device.  One copy of
+// contiguous memory: strided 2-D copies into pageable memory returned stale
+// rows when a profiler was attached.
+static int copy_block(gvh_context *c, const void *block, bool is_float, bool all, double *host) {
+  const size_t n = all ? (size_t)c->G : (size_t)c->nx * c->ny * c->nz;
+  const void *src = block;
+  if (is_float || !all) {
+    HIP_TRY(launch_pack(block, is_float, extent_of(c), all, transfer_scratch(c), c->stream));
+    src = transfer_scratch(c);
   }
-  HIP_TRY(hipMemcpyAsync(host, qbase + f * G, G * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(hipMemcpyAsync(host, src, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
   return GVH_OK;
+}
+
+int gvh_copy_q_field(gvh_context *c, const double *qbase, int f, double *host) {
+  const size_t G = (size_t)c->G;
+  if (c->precision != GVH_FP64 && f >= GVH_PITT)
+    return copy_block(c, reinterpret_cast<const float *>(qbase + 4 * G) + (f - GVH_PITT) * G, true,
+                      true, host);
+  return copy_block(c, qbase + f * G, false, true, host);
 }
 
 extern "C" int gvh_set_field(gvh_context *c, int field, const double *host_ghosted) {
@@ -500,44 +478,11 @@ extern "C" int gvh_get_field(gvh_context *c, int field, int ghosted, double *hos
   bool fl;
   void *dv = field_dev(c, field, &fl);
   if (!dv) return gvh_fail(GVH_EINVAL, "unknown field %d", field);
-  if (fl) {
-    std::vector<double> full(c->G);
-    int rc = gvh_copy_q_field(c, c->qbuf[c->iq], field, full.data());
-    if (rc) return rc;
-    if (ghosted) {
-      std::copy(full.begin(), full.end(), host_out);
-    } else {
-      for (int k = 0; k < c->nz; ++k)
-        for (int j = 0; j < c->ny; ++j)
-          for (int i = 0; i < c->nx; ++i)
-            host_out[i + (size_t)c->nx * (j + (size_t)c->ny * k)] =
-                full[(i + 2) + (size_t)c->ncx * ((j + 2) + (size_t)c->ncy * (k + 2))];
-    }
-    return GVH_OK;
-  }
-  return gvh_copy_ghosted_field(c, (const double *)dv, ghosted, host_out);
+  return copy_block(c, dv, fl, ghosted != 0, host_out);
 }
 
-// One ghosted block of G doubles to the host: the whole block with one copy,
-// then (ghosted == 0) the interior cells picked on the host.  Strided 2-D
-// copies into pageable memory returned stale rows when a profiler was
-// attached, so none are used.
 int gvh_copy_ghosted_field(gvh_context *c, const double *d, int ghosted, double *host_out) {
-  if (ghosted) {
-    HIP_TRY(hipMemcpyAsync(host_out, d, (size_t)c->G * sizeof(double), hipMemcpyDeviceToHost,
-                           c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return GVH_OK;
-  }
-  std::vector<double> full(c->G);
-  HIP_TRY(hipMemcpyAsync(full.data(), d, (size_t)c->G * sizeof(double), hipMemcpyDeviceToHost,
-                         c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  for (int k = 0; k < c->nz; ++k)
-    for (int j = 0; j < c->ny; ++j)
-      std::copy_n(full.data() + 2 + (size_t)c->ncx * ((j + 2) + (size_t)c->ncy * (k + 2)), c->nx,
-                  host_out + (size_t)c->nx * (j + (size_t)c->ny * k));
-  return GVH_OK;
+  return copy_block(c, d, false, ghosted != 0, host_out);
 }
 
 // Arguments of one stage launch for the current buffer roles.
