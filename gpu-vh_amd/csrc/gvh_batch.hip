@@ -131,6 +131,7 @@ double seconds(Clock::time_point a, Clock::time_point b) {
 }  // namespace
 
 struct gvh_batch {
+  gvh::Staging staging;  // of the events' contexts
   gvh_options opts{};
   std::vector<double> tab_p, tab_cs2, tab_T;
   hipStream_t stream = nullptr;
@@ -469,6 +470,7 @@ int admit(gvh_batch *b) {
       b->queue.pop_front();
       continue;
     }
+    c->staging = &b->staging;
     if (P.newton_budget > 0 && P.newton_budget < MAX_ITERS) c->max_iters = P.newton_budget;
     const size_t n = P.e.size();
     std::vector<double> p(n), ut(n, 1.0), zero(n, 0.0);

