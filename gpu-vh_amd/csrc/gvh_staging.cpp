@@ -3,6 +3,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cstdint>
 #include <cstring>
 #include <thread>
 #include <vector>
@@ -10,6 +11,8 @@
 namespace gvh {
 
 namespace {
+
+constexpr int CHUNK_BLOCKS = 32;
 
 // Pinned (or device) memory that the runtime copies to and from directly.
 bool is_pinned(const void *p) {
@@ -24,8 +27,7 @@ bool is_pinned(const void *p) {
 }  // namespace
 
 Staging::~Staging() {
-  for (hipEvent_t e : ev_)
-    if (e) (void)hipEventDestroy(e);
+  if (arrived_) (void)hipFree(arrived_);
   if (mem_) (void)hipHostFree(mem_);
   if (small_) (void)hipHostFree(small_);
 }
@@ -41,11 +43,13 @@ void *Staging::small(size_t bytes) {
 
 bool Staging::ready() {
   if (mem_ || failed_) return mem_ != nullptr;
-  bool ok = true;
-  for (hipEvent_t &e : ev_)
-    if (!e) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
-  ok = ok && hipHostMalloc((void **)&mem_, NSLOT * SLOT) == hipSuccess;
+  bool ok = hipHostMalloc((void **)&mem_, NSLOT * SLOT + sizeof(unsigned) * NSLOT,
+                          hipHostMallocCoherent) == hipSuccess;
+  ok = ok && hipMalloc((void **)&arrived_, sizeof(unsigned) * NSLOT) == hipSuccess;
+  ok = ok && hipMemset(arrived_, 0, sizeof(unsigned) * NSLOT) == hipSuccess &&
+       hipStreamSynchronize(nullptr) == hipSuccess;
   if (!ok) {
+    if (mem_) (void)hipHostFree(mem_);
     (void)hipGetLastError();
     mem_ = nullptr;
     failed_ = true;
@@ -53,10 +57,31 @@ bool Staging::ready() {
   return ok;
 }
 
-// Chunks of SLOT bytes go round the slots.  The calling thread issues the
-// device copies and waits for their events; it and the others each copy their
-// share of a chunk from its slot.  `open` counts the chunks that have arrived,
-// done[c] the shares of chunk c that are copied.
+// One chunk of 4-byte words into its slot; the last block to have its part
+// there tells the host.  16-byte stores where the chunk's start allows them:
+// its words from `n4` 16-byte groups on go one by one.
+__global__ __launch_bounds__(256) void chunk_kernel(const unsigned *__restrict__ src,
+                                                    unsigned *__restrict__ slot, unsigned words,
+                                                    unsigned n4, unsigned *__restrict__ arrived,
+                                                    unsigned *__restrict__ flag) {
+  const unsigned t = blockIdx.x * 256 + threadIdx.x, nt = gridDim.x * 256;
+  for (unsigned i = t; i < n4; i += nt)
+    reinterpret_cast<uint4 *>(slot)[i] = reinterpret_cast<const uint4 *>(src)[i];
+  for (unsigned i = 4 * n4 + t; i < words; i += nt) slot[i] = src[i];
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0 && atomicAdd(arrived, 1u) == gridDim.x - 1) {
+    *arrived = 0;
+    __hip_atomic_store(flag, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+// Chunks of SLOT bytes go round the slots.  The calling thread launches their
+// kernels and waits for their flags; it and the others each copy their share
+// of a chunk from its slot.  `open` counts the chunks that have arrived,
+// done[c] the shares of chunk c that are copied.  (With the runtime's copies
+// and events instead, a thread of the runtime stays busy for milliseconds
+// afterwards, and a program whose threads fill the CPUs waits for it.)
 hipError_t Staging::pipeline(char *host, const char *dev, size_t bytes, hipStream_t st) {
   const int n = (int)((bytes + SLOT - 1) / SLOT);
   const int nt = std::max(1, std::min({MAX_THREADS, n, (int)std::thread::hardware_concurrency()}));
@@ -93,15 +118,29 @@ hipError_t Staging::pipeline(char *host, const char *dev, size_t bytes, hipStrea
     while (done[c].load(std::memory_order_acquire) < threads) std::this_thread::yield();
   };
   hipError_t e = hipSuccess;
+  unsigned *flags = reinterpret_cast<unsigned *>(mem_ + NSLOT * SLOT);
+  auto set = [&](int c) { return __atomic_load_n(flags + c % NSLOT, __ATOMIC_ACQUIRE) != 0u; };
   int issued = 0;
   for (int c = 0; c < n && e == hipSuccess; ++c) {
     for (; issued < n && issued < c + NSLOT && e == hipSuccess; ++issued) {
       if (issued >= NSLOT) finish(issued - NSLOT);
-      e = hipMemcpyAsync(mem_ + (size_t)(issued % NSLOT) * SLOT, dev + (size_t)issued * SLOT,
-                         length(issued), hipMemcpyDeviceToHost, st);
-      if (e == hipSuccess) e = hipEventRecord(ev_[issued % NSLOT], st);
+      const int k = issued % NSLOT;
+      const char *src = dev + (size_t)issued * SLOT;
+      const unsigned words = (unsigned)(length(issued) / 4);
+      __atomic_store_n(flags + k, 0u, __ATOMIC_RELEASE);
+      chunk_kernel<<<CHUNK_BLOCKS, 256, 0, st>>>(
+          reinterpret_cast<const unsigned *>(src), reinterpret_cast<unsigned *>(mem_ + k * SLOT), words,
+          reinterpret_cast<uintptr_t>(src) % 16 == 0 ? words / 4 : 0u, arrived_ + k, flags + k);
+      e = hipGetLastError();
     }
-    if (e == hipSuccess) e = hipEventSynchronize(ev_[c % NSLOT]);
+    // the stream tells of a failed kernel, whose flag would never come
+    for (int polls = 1; e == hipSuccess && !set(c); ++polls) {
+      if (polls % 4096 == 0) {
+        const hipError_t q = hipStreamQuery(st);
+        if (q == hipSuccess && !set(c)) e = hipErrorUnknown;
+        else if (q != hipSuccess && q != hipErrorNotReady) e = q;
+      }
+    }
     if (e != hipSuccess) break;
     open.store(c + 1, std::memory_order_release);
     share(c, 0);
@@ -115,7 +154,7 @@ hipError_t Staging::pipeline(char *host, const char *dev, size_t bytes, hipStrea
 }
 
 hipError_t Staging::to_host(void *host, const void *dev, size_t bytes, hipStream_t st) {
-  if (bytes >= SLOT && !is_pinned(host) && ready()) {
+  if (bytes >= SLOT && bytes % 4 == 0 && !is_pinned(host) && ready()) {
     try {
       return pipeline(static_cast<char *>(host), static_cast<const char *>(dev), bytes, st);
     } catch (...) {  // no memory for its bookkeeping, before anything was issued

@@ -2,10 +2,11 @@
 //
 // The runtime moves pageable memory to the host at 17 GB/s on one core, 5 to
 // 8 GB/s where the caller's pages are new, over a link that does 57.  Here large
-// results come through pinned slots of 1 MiB that four threads empty, so the
-// link, the copies and the page faults overlap: into new pages 1.7 MB take 120
-// against 250 us, 4.2 MB 320 against 550, 33 MB 1.4 against 6.9 ms (slots of 512
-// KiB: 190, 390 us, 1.8 ms; six threads: 115, 480 us, 1.4 ms).  Copies to the
+// results come through pinned slots of 1 MiB that a kernel fills and four
+// threads empty, so the link, the copies and the page faults overlap: into new
+// pages 1.7 MB take 120 against 250 us, 4.2 MB 320 against 550, 33 MB 1.25
+// against 6.9 ms (with the runtime's copies into the slots 1.4 ms; slots of 512
+// KiB 1.8 ms; six threads 480 us for 4.2 MB).  Copies to the
 // device gain nothing by it: the runtime reads pageable memory at 30 GB/s.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -36,9 +37,10 @@ class Staging {
  private:
   bool ready();
   hipError_t pipeline(char *host, const char *dev, size_t bytes, hipStream_t st);
-  char *mem_ = nullptr, *small_ = nullptr;
+  char *mem_ = nullptr;  // the slots, then a flag for each
+  char *small_ = nullptr;
   bool failed_ = false;
-  hipEvent_t ev_[NSLOT] = {};
+  unsigned *arrived_ = nullptr;  // per slot, blocks that have their part there
 };
 
 }  // namespace gvh
