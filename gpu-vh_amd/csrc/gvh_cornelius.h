@@ -686,50 +686,134 @@ __device__ __forceinline__ double third(double x) {
   return fma(fma(-3.0, q, x), r, q);
 }
 
+// 1 / (2 n) for a polygon of n = 3..6 lines, and x / (2 n) from it, correctly
+// rounded in the same way.
+__device__ __forceinline__ double one_over_twice(int n) {
+  int hi = n == 3 ? 0x3fc55555 : (n == 4 ? 0x3fc00000 : (n == 5 ? 0x3fb99999 : 0x3fb55555));
+  int lo = n == 4 ? 0 : (n == 5 ? (int)0x9999999au : 0x55555555);
+  // the words stay selects; seen as a double, they become four branches
+  asm("" : "+v"(hi), "+v"(lo));
+  return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double over_twice(double x, int n, double r) {
+  const double q = x * r;
+  return fma(fma(-double(2 * n), q, x), r, q);
+}
+
+// x / b, correctly rounded, from r = 1 / b correctly rounded: one residual
+// correction makes the quotient faithful, a second one exact.
+__device__ __forceinline__ double quotient(double x, double b, double r) {
+  double q = x * r;
+  q = fma(fma(-b, q, x), r, q);
+  return fma(fma(-b, q, x), r, q);
+}
+
 // Squares of a cell: number 6 q + r, q = 2 a + j the cube that holds axis a
 // at side j, r = 2 f + jj its square that holds the cube's f-th free axis at
 // side jj.  A 3-D cell is the cube q = 0 with corners 0..7.
 struct SquareInfo {
-  unsigned base, w1, w2;    // corner (0, 0); corner weights of the free axes
-  unsigned x1, x2, a, xf;   // free axes x1 < x2, held axes
-  unsigned j, jj;           // sides of a and xf
-  unsigned i0, i1, i2, i3;  // edges (x2 = 0), (x1 = 0), (x1 = h1), (x2 = h2)
+  unsigned base, w1, w2;  // corner (0, 0); corner weights of the free axes
+  unsigned x1, x2;        // free axes x1 < x2
+  unsigned edge[4];       // edges (x2 = 0), (x1 = 0), (x1 = h1), (x2 = h2)
 };
 // Edge number: axis * 8 + the corner's sides along the other axes.
-__device__ __forceinline__ unsigned edge_number(unsigned d, unsigned corner) {
+__host__ __device__ constexpr unsigned edge_number(unsigned d, unsigned corner) {
   return d * 8 + ((corner >> (4 - d)) << (3 - d) | (corner & ((8u >> d) - 1u)));
 }
-__device__ __forceinline__ uint2 pack_square(unsigned n) {
+__host__ __device__ constexpr SquareInfo square_info(unsigned n) {
   const unsigned q = n / 6, r = n - 6 * q, a = q >> 1, j = q & 1, f = r >> 1, jj = r & 1;
-  auto axis = [&](unsigned i) { return i + (i >= a ? 1u : 0u); };
-  const unsigned xf = axis(f), x1 = axis(f == 0 ? 1 : 0), x2 = axis(f == 2 ? 1 : 2);
+  const unsigned i1 = f == 0 ? 1 : 0, i2 = f == 2 ? 1 : 2;
+  const unsigned xf = f + (f >= a ? 1u : 0u), x1 = i1 + (i1 >= a ? 1u : 0u), x2 = i2 + (i2 >= a ? 1u : 0u);
   const unsigned base = j * (8u >> a) + jj * (8u >> xf), w1 = 8u >> x1, w2 = 8u >> x2;
-  return uint2{base | w1 << 4 | w2 << 8 | x1 << 12 | x2 << 14 | a << 16 | xf << 18 | j << 20 | jj << 21,
-               edge_number(x1, base) | edge_number(x2, base) << 5 |
-                   edge_number(x2, base + w1) << 10 | edge_number(x1, base + w2) << 15};
-}
-__device__ __forceinline__ SquareInfo unpack_square(uint2 p) {
-  return SquareInfo{p.x & 15u,         (p.x >> 4) & 15u,  (p.x >> 8) & 15u,  (p.x >> 12) & 3u,
-                    (p.x >> 14) & 3u,  (p.x >> 16) & 3u,  (p.x >> 18) & 3u,  (p.x >> 20) & 1u,
-                    (p.x >> 21) & 1u,  p.y & 31u,         (p.y >> 5) & 31u,  (p.y >> 10) & 31u,
-                    (p.y >> 15) & 31u};
+  return SquareInfo{base, w1, w2, x1, x2,
+                    {edge_number(x1, base), edge_number(x2, base), edge_number(x2, base + w1),
+                     edge_number(x1, base + w2)}};
 }
 // Corners (0,0), (0,1), (1,0), (1,1) of a square above v0, as bits 0..3.
-__device__ __forceinline__ unsigned square_bits(const SquareInfo &q, unsigned m) {
-  const unsigned b = m >> q.base;
-  return (b & 1u) | ((b >> q.w2) & 1u) << 1 | ((b >> q.w1) & 1u) << 2 |
-         ((b >> (q.w1 + q.w2)) & 1u) << 3;
+__host__ __device__ constexpr unsigned square_bits(unsigned base, unsigned w1, unsigned w2, unsigned m) {
+  const unsigned b = m >> base;
+  return (b & 1u) | ((b >> w2) & 1u) << 1 | ((b >> w1) & 1u) << 2 | ((b >> (w1 + w2)) & 1u) << 3;
 }
-// First and last cut edge (0..3) of a square with two cuts.
-__device__ __forceinline__ void cut_edges(unsigned sq, unsigned &first, unsigned &last) {
-  const bool c0 = ((sq >> 2) ^ sq) & 1u, c1 = ((sq >> 1) ^ sq) & 1u;
-  const bool c2 = ((sq >> 3) ^ (sq >> 2)) & 1u, c3 = ((sq >> 3) ^ (sq >> 1)) & 1u;
-  first = c0 ? 0 : (c1 ? 1 : 2);
-  last = c3 ? 3 : (c2 ? 2 : 1);
+
+// What the pattern of a cube's eight corners says of it: its lines in the
+// order and direction in which the general search joins them, each as start
+// edge | end edge << 5 | square << 10.
+struct alignas(16) CubeLines {
+  unsigned short line[6];
+  unsigned info;  // number of lines; flags; the squares that are cut << 8
+};
+constexpr unsigned CUBE_NLINES = 7u, CUBE_NOT_PLAIN = 8u, CUBE_HEXAGON = 16u;
+struct CubePatterns {
+  CubeLines p[256];
+};
+constexpr CubePatterns cube_patterns(unsigned q) {
+  CubePatterns T{};
+  const unsigned a = q >> 1;
+  SquareInfo sq[6] = {};
+  for (unsigned r = 0; r < 6; ++r) sq[r] = square_info(6 * q + r);
+  for (unsigned pat = 0; pat < 256; ++pat) {
+    // the cell's corners on this cube
+    unsigned m = 0, above = 0;
+    for (unsigned i = 0; i < 8; ++i) {
+      const unsigned low = i & ((8u >> a) - 1u), c = (i - low) << 1 | (q & 1 ? 8u >> a : 0u) | low;
+      m |= ((pat >> i) & 1u) << c;
+      above += (pat >> i) & 1u;
+    }
+    unsigned first[6] = {}, last[6] = {}, cut = 0, n = 0;
+    bool crossed = false;
+    for (unsigned r = 0; r < 6; ++r) {
+      const unsigned b = square_bits(sq[r].base, sq[r].w1, sq[r].w2, m);
+      if (b == 0 || b == 15) continue;
+      if (b == 6 || b == 9) crossed = true;
+      const unsigned c[4] = {((b >> 2) ^ b) & 1u, ((b >> 1) ^ b) & 1u, ((b >> 3) ^ (b >> 2)) & 1u,
+                             ((b >> 3) ^ (b >> 1)) & 1u};
+      first[r] = sq[r].edge[c[0] ? 0 : (c[1] ? 1 : 2)];
+      last[r] = sq[r].edge[c[3] ? 3 : (c[2] ? 2 : 1)];
+      cut |= 1u << r;
+      ++n;
+    }
+    CubeLines &L = T.p[pat];
+    // two opposite corners apart from the six others: two triangles
+    if (crossed || (n == 6 && (above == 2 || above == 6))) {
+      L.info = CUBE_NOT_PLAIN;
+      continue;
+    }
+    L.info = n | (n == 6 ? CUBE_HEXAGON : 0u) | cut << 8;
+    unsigned left = cut, end = 0;
+    for (unsigned k = 0; k < n; ++k) {
+      unsigned r = 0;
+      while (!((left >> r) & 1u)) ++r;
+      bool turned = false;
+      if (n == 6 && k > 0) {
+        // around the hexagon: the first line left that begins or ends here
+        while (!(((left >> r) & 1u) && (first[r] == end || last[r] == end))) ++r;
+        turned = last[r] == end;
+      }
+      left &= ~(1u << r);
+      end = turned ? first[r] : last[r];
+      L.line[k] = (unsigned short)((turned ? last[r] : first[r]) | end << 5 | (6 * q + r) << 10);
+    }
+  }
+  return T;
 }
-__device__ __forceinline__ unsigned pick4(unsigned k, unsigned a, unsigned b, unsigned c,
-                                          unsigned d) {
-  return k == 0 ? a : (k == 1 ? b : (k == 2 ? c : d));
+constexpr CubePatterns CUBE0 = cube_patterns(0), CUBE1 = cube_patterns(1), CUBE2 = cube_patterns(2),
+                       CUBE3 = cube_patterns(3), CUBE4 = cube_patterns(4), CUBE5 = cube_patterns(5),
+                       CUBE6 = cube_patterns(6), CUBE7 = cube_patterns(7);
+__device__ const CubePatterns CUBES[8] = {CUBE0, CUBE1, CUBE2, CUBE3, CUBE4, CUBE5, CUBE6, CUBE7};
+
+// The eight corners of the cube that holds axis a at side j, as bits.
+__device__ __forceinline__ unsigned cube_corners(unsigned m, unsigned a, unsigned j) {
+  unsigned x = m >> (j * (8u >> a));
+  if (a == 0) return x & 255u;
+  if (a == 1) return (x & 15u) | ((x >> 4) & 0xf0u);
+  if (a == 3) {
+    x &= 0x5555u;
+    x = (x | x >> 1) & 0x3333u;
+  } else {
+    x &= 0x3333u;
+  }
+  x = (x | x >> 2) & 0x0f0fu;
+  return (x | x >> 4) & 255u;
 }
 
 // LDS of a wave of plain cells; columns are lanes.  A line in the list is its
@@ -740,12 +824,43 @@ struct PlainLds {
   double E[32 * 64];                     // edge cuts
   double pc[DIM == 4 ? 8 * D * 64 : 1];  // polygon centroids, by cube
   double2 at[32][2];                     // position of an edge: its held coordinates
-  uint2 sq[48];
-  unsigned short list[LINES * 64];       // start edge | end edge << 5 | square << 10
+  double mean[5][4];                     // by class and axis: mean of corners below v0
+  unsigned sq[48];                       // base | w1 << 4 | w2 << 8 | x1 << 12 | x2 << 14
+  unsigned short list[(LINES + 1) * 64]; // start edge | end edge << 5 | square << 10; a row to spare
 };
+
+// Mean of the corners of a square below v0 along one of its free axes, of
+// length h, by how many of them lie on the far side and how many there are:
+// 0, h/2, h, h/3, 2h/3 (classes 0..4; MEAN_CLASS1 and 2 hold those of the
+// square's two axes, three bits for each pattern of corners below).
+__device__ __forceinline__ double class_mean(unsigned k, double h) {
+  return k == 0 ? 0.0 : (k == 1 ? 0.5 * h : (k == 2 ? h : third(k == 3 ? h : h + h)));
+}
+constexpr unsigned long long mean_classes(unsigned far) {
+  unsigned long long t = 0;
+  for (unsigned low = 1; low < 15; ++low) {
+    unsigned n = 0, n1 = 0;
+    for (unsigned i = 0; i < 4; ++i) {
+      n += (low >> i) & 1u;
+      n1 += ((low & far) >> i) & 1u;
+    }
+    const unsigned k = n1 == 0 ? 0 : (n == 3 ? 2 + n1 : (n == 2 && n1 == 1 ? 1 : 2));
+    t |= (unsigned long long)k << (3 * low);
+  }
+  return t;
+}
+constexpr unsigned long long MEAN_CLASS1 = mean_classes(12u), MEAN_CLASS2 = mean_classes(10u);
+
 template <int DIM>
 __device__ __forceinline__ void plain_tables(PlainLds<DIM> &S, int lane, const double *h) {
-  if (lane < (DIM == 4 ? 48 : 6)) S.sq[lane] = pack_square(lane);
+  if (lane < (DIM == 4 ? 48 : 6)) {
+    const SquareInfo q = square_info(lane);
+    S.sq[lane] = q.base | q.w1 << 4 | q.w2 << 8 | q.x1 << 12 | q.x2 << 14;
+  }
+  if (lane < 20) {
+    const unsigned x = lane & 3u;
+    S.mean[lane >> 2][x] = class_mean(lane >> 2, x == 0 ? h[0] : (x == 1 ? h[1] : (x == 2 ? h[2] : h[3])));
+  }
   if (lane < 32) {
     const unsigned d = lane >> 3, pos = lane & 7u;
     const unsigned c = (pos >> (3 - d)) << (4 - d) | (pos & ((8u >> d) - 1u));
@@ -777,176 +892,110 @@ __device__ __forceinline__ Line4 plain_line(const PlainLds<DIM> &S, int lane, un
   return l;
 }
 // body(line, id, whether it is a polygon's last) for the lines of the lane's
-// list; bit i of ends is set for a polygon's last line.  The next line is
-// fetched while the body works on this one: a line is two dependent LDS reads,
-// and few waves fit a CU to hide them.
+// list; bit i of ends is set for a polygon's last line.  The next line and the
+// number of the one after it are fetched while the body works on this one: a
+// line is two dependent LDS reads, and few waves fit a CU to hide them.
 template <int DIM, typename B>
 __device__ __forceinline__ void for_lines(const PlainLds<DIM> &S, int lane, int nl,
                                           unsigned long long ends, B &&body) {
-  unsigned id = S.list[lane];
+  auto number = [&](int i) -> unsigned { return S.list[64 * (i < nl ? i : 0) + lane]; };
+  unsigned id = number(0), idn = number(1);
   Line4 l = plain_line(S, lane, id);
 #pragma unroll 1
-  for (int i = 1; i <= nl; ++i) {
-    const unsigned idn = S.list[64 * (i < nl ? i : 0) + lane];
+  for (int i = 2; i <= nl + 1; ++i) {
+    const unsigned idnn = number(i);
     const Line4 ln = plain_line(S, lane, idn);
     body(l, id, (bool)(ends & 1ull));
     ends >>= 1;
     l = ln;
     id = idn;
+    idn = idnn;
   }
 }
 
-// Mean of the corners below v0 along one free axis of length h: n1 of nout
-// lie on the far side.
-__device__ __forceinline__ double outside_mean(int n1, int nout, double h) {
-  const double x = n1 == 0 ? 0.0 : (n1 == 2 ? h + h : h);
-  return nout == 1 ? x : (nout == 2 ? 0.5 * x : third(x));
-}
 // Outside point of a line (outside() of the general search).
 template <int DIM>
 __device__ __forceinline__ void plain_outside(const PlainLds<DIM> &S, unsigned id, unsigned m,
-                                              const double *h, const double *s, double *o) {
-  const SquareInfo q = unpack_square(S.sq[id >> 10]);
-  const unsigned low = ~square_bits(q, m) & 15u;
-  const int nout = __popc(low);
-  const double g0 = h[0], g1 = h[1], g2 = h[2], g3 = h[3];
-  const double h1 = q.x1 == 0 ? g0 : (q.x1 == 1 ? g1 : g2);
-  const double h2 = q.x2 == 1 ? g1 : (q.x2 == 2 ? g2 : g3);
-  const double o1 = outside_mean(__popc(low & 12u), nout, h1);
-  const double o2 = outside_mean(__popc(low & 10u), nout, h2);
+                                              const double *s, double *o) {
+  const unsigned q = S.sq[id >> 10], x1 = (q >> 12) & 3u, x2 = q >> 14;
+  const unsigned low = ~square_bits(q & 15u, (q >> 4) & 15u, (q >> 8) & 15u, m) & 15u;
+  const double o1 = S.mean[(unsigned)(MEAN_CLASS1 >> (3 * low)) & 7u][x1];
+  const double o2 = S.mean[(unsigned)(MEAN_CLASS2 >> (3 * low)) & 7u][x2];
 #pragma unroll
-  for (unsigned k = 0; k < D; ++k) o[k] = k == q.x1 ? o1 : (k == q.x2 ? o2 : s[k]);
+  for (unsigned k = 0; k < D; ++k) o[k] = k == x1 ? o1 : (k == x2 ? o2 : s[k]);
 }
 
-// Lines of the hexagon of cube q in the order and direction in which the
-// general search joins them, into the list from pos on.
-template <int DIM>
-__device__ __forceinline__ void list_hexagon(PlainLds<DIM> &S, int lane, unsigned m, unsigned q,
-                                             unsigned pos) {
-  unsigned first = 0, last = 0;  // edge numbers of the six lines, five bits each
-#pragma unroll 1
-  for (unsigned r = 0; r < 6; ++r) {
-    const SquareInfo i = unpack_square(S.sq[6 * q + r]);
-    unsigned f, l;
-    cut_edges(square_bits(i, m), f, l);
-    first |= pick4(f, i.i0, i.i1, i.i2, i.i3) << (5 * r);
-    last |= pick4(l, i.i0, i.i1, i.i2, i.i3) << (5 * r);
-  }
-  unsigned end = last & 31u, free = 62u;
-  S.list[64 * pos + lane] = (unsigned short)((first & 31u) | end << 5 | (6 * q) << 10);
-#pragma unroll 1
-  for (unsigned k = 1; k < 6; ++k) {
-    unsigned next = 0, turned = 0;
-#pragma unroll
-    for (unsigned r = 5; r >= 1; --r)
-      if ((free >> r) & 1u) {
-        const bool sm = ((first >> (5 * r)) & 31u) == end, em = ((last >> (5 * r)) & 31u) == end;
-        if (sm || em) {
-          next = r;
-          turned = em ? 1u : 0u;
-        }
-      }
-    const unsigned start = ((turned ? last : first) >> (5 * next)) & 31u;
-    end = ((turned ? first : last) >> (5 * next)) & 31u;
-    free &= ~(1u << next);
-    S.list[64 * (pos + k) + lane] = (unsigned short)(start | end << 5 | (6 * q + next) << 10);
-  }
-}
-
-// Squares of the cell that are cut, and whether one is cut four times.
-template <int DIM>
-__device__ __forceinline__ unsigned long long cut_squares(unsigned m, bool &crossed) {
-  constexpr int NQ = DIM == 4 ? 8 : 1;
-  unsigned long long cut = 0;
-  crossed = false;
-#pragma unroll
-  for (unsigned q = 0; q < NQ; ++q)
-#pragma unroll
-    for (unsigned r = 0; r < 6; ++r) {
-      const unsigned a = q >> 1, f = r >> 1;
-      auto axis = [&](unsigned i) { return i + (i >= a ? 1u : 0u); };
-      const unsigned x1 = axis(f == 0 ? 1 : 0), x2 = axis(f == 2 ? 1 : 2), w1 = 8u >> x1, w2 = 8u >> x2;
-      const unsigned base = (q & 1) * (8u >> a) + (r & 1) * (8u >> axis(f));
-      const unsigned sel = (1u | 1u << w1 | 1u << w2 | 1u << (w1 + w2)) << base;
-      const unsigned in = m & sel;
-      const unsigned d1 = (1u | 1u << (w1 + w2)) << base, d2 = (1u << w1 | 1u << w2) << base;
-      if (in != 0u && in != sel) cut |= 1ull << (6 * q + r);
-      crossed = crossed || in == d1 || in == d2;
-    }
-  return cut;
-}
-
-// Lists the lines of the lane's cell (corner pattern m, edge cuts in S.E;
-// near: one of them within 1e-10 of a corner); the number of lines, or 0 if
-// the cell is not plain.  ends: the last lines of polygons.
+// Lists the lines of the lane's cell (corner pattern m; near: an edge cut
+// within 1e-10 of a corner); the number of lines, or 0 if the cell is not
+// plain.  ends: the last lines of polygons.  The eight cubes are looked up
+// together and written without branches: following the lines of one cube
+// after another, each lane through its own cubes, took 24 000 cycles of a
+// window's 188 000 per wave, and 56 000 where one cell in ten has a hexagon.
 template <int DIM>
 __device__ __forceinline__ int list_lines(PlainLds<DIM> &S, int lane, unsigned m, bool near,
                                           unsigned long long &ends) {
   constexpr unsigned NQ = DIM == 4 ? 8 : 1;
-  bool crossed;
-  const unsigned long long cut = cut_squares<DIM>(m, crossed);
-  if (crossed) return 0;
-  auto lines = [&](unsigned q) { return (unsigned)(cut >> (6 * q)) & 63u; };
-  unsigned present = 0, hexagons = 0;
+  CubeLines c[NQ];
+#pragma unroll
+  for (unsigned q = 0; q < NQ; ++q) c[q] = CUBES[q].p[cube_corners(m, q >> 1, q & 1)];
+  unsigned any = 0, present = 0, nlines = 0;
 #pragma unroll
   for (unsigned q = 0; q < NQ; ++q) {
-    const unsigned f = lines(q);
-    present |= (f ? 1u : 0u) << q;
-    hexagons |= (f == 63u ? 1u : 0u) << q;
-    if (f == 63u) {
-      // two opposite corners apart from the six others: two triangles
-      const unsigned a = q >> 1, w = 8u >> a;
-      unsigned side = 0;
-#pragma unroll
-      for (unsigned c = 0; c < 16; ++c)
-        if ((c & w) == ((q & 1) ? w : 0u)) side |= 1u << c;
-      const int n = __popc(m & side);
-      if (n == 2 || n == 6) return 0;
-    }
+    const unsigned n = c[q].info & CUBE_NLINES;
+    any |= c[q].info;
+    present |= (n ? 1u : 0u) << q;
+    nlines += n;
   }
-  const int nlines = __popcll(cut), na = __popc(m), few = na < 16 - na ? na : 16 - na;
-  bool joined = hexagons != 0u;
-  if constexpr (DIM == 4) joined = joined || (nlines == 24 && few == 2);
+  if (any & CUBE_NOT_PLAIN) return 0;
+  bool joined = any & CUBE_HEXAGON;
+  if constexpr (DIM == 4) {
+    const int na = __popc(m);
+    joined = joined || (nlines == 24 && (na == 2 || na == 14));
+  }
   if (joined && near) return 0;
-  unsigned taken = 0, pos = 0;
-  ends = 0;
-#pragma unroll 1
-  for (unsigned t = 0; t < NQ; ++t) {
-    unsigned next = present & ~taken;
-    if (joined && taken) {
-      unsigned touch = 0;
+  unsigned pos[NQ];  // of the cube's first line
+  unsigned at = 0;
+#pragma unroll
+  for (unsigned q = 0; q < NQ; ++q) {
+    pos[q] = at;
+    at += c[q].info & CUBE_NLINES;
+  }
+  if constexpr (DIM == 4)
+    if (joined) {
+      // cubes in the order in which they touch those before, the lowest first:
+      // bytes by cube of the cubes that share a cut square with it (the held
+      // axes of its cut squares) and of its lines; bytes by cube of positions
+      unsigned long long touching = 0, lengths = 0, posq = 0;
 #pragma unroll
       for (unsigned q = 0; q < NQ; ++q) {
-        // cubes that share a cut square with q: its squares' held axes
-        const unsigned f = lines(q), a2 = q & ~1u;
-        const unsigned adj = (f & ((1u << a2) - 1u)) | (f >> a2) << (a2 + 2);
-        touch |= (adj & taken ? 1u : 0u) << q;
+        const unsigned f = (c[q].info >> 8) & 63u, a2 = q & ~1u;
+        touching |= (unsigned long long)((f & ((1u << a2) - 1u)) | (f >> a2) << (a2 + 2)) << (8 * q);
+        lengths |= (unsigned long long)(c[q].info & CUBE_NLINES) << (8 * q);
       }
-      next &= touch;
-    }
-    if (!next) break;
-    const unsigned q = (unsigned)__builtin_ctz(next);
-    taken |= 1u << q;
-    if ((hexagons >> q) & 1u) {
-      list_hexagon(S, lane, m, q, pos);
-      pos += 6;
-    } else {
-      unsigned f = (unsigned)(cut >> (6 * q)) & 63u;
-      while (f) {
-        const unsigned r = (unsigned)__builtin_ctz(f);
-        f &= f - 1u;
-        const SquareInfo i = unpack_square(S.sq[6 * q + r]);
-        unsigned a, z;
-        cut_edges(square_bits(i, m), a, z);
-        S.list[64 * pos + lane] =
-            (unsigned short)(pick4(a, i.i0, i.i1, i.i2, i.i3) |
-                             pick4(z, i.i0, i.i1, i.i2, i.i3) << 5 | (6 * q + r) << 10);
-        ++pos;
+      unsigned left = present, touch = 255u;
+      at = 0;
+#pragma unroll 1
+      while (left & touch) {
+        const unsigned q = (unsigned)__builtin_ctz(left & touch);
+        posq |= (unsigned long long)at << (8 * q);
+        at += (unsigned)(lengths >> (8 * q)) & 255u;
+        touch = (left == present ? 0u : touch) | ((unsigned)(touching >> (8 * q)) & 255u);
+        left &= ~(1u << q);
       }
+      if (left) return 0;
+#pragma unroll
+      for (unsigned q = 0; q < NQ; ++q) pos[q] = (unsigned)(posq >> (8 * q)) & 255u;
     }
-    ends |= 1ull << (pos - 1);
+  ends = 0;
+#pragma unroll
+  for (unsigned q = 0; q < NQ; ++q) {
+    const unsigned n = c[q].info & CUBE_NLINES;
+    if constexpr (DIM == 4) ends |= n ? 1ull << (pos[q] + n - 1) : 0ull;
+#pragma unroll
+    for (unsigned k = 0; k < 6; ++k)
+      S.list[64 * (k < n ? pos[q] + k : (unsigned)PlainLds<DIM>::LINES) + lane] = c[q].line[k];
   }
-  return taken == present ? (int)pos : 0;
+  return (int)nlines;
 }
 
 // Element of the lane's plain 4-D cell of nl lines.  The sums are those of
@@ -966,8 +1015,9 @@ __device__ __forceinline__ void plain_element4(PlainLds<4> &S, int lane, unsigne
     }
     ++n;
     if (last) {
+      const double r = one_over_twice(n);
       for (int k = 0; k < D; ++k) {
-        pc(id, k) = pm[k] / double(2.0 * n);
+        pc(id, k) = over_twice(pm[k], n, r);
         pm[k] = 0;
       }
       n = 0;
@@ -998,8 +1048,10 @@ __device__ __forceinline__ void plain_element4(PlainLds<4> &S, int lane, unsigne
     down += ar;
     ++n;
     if (last) {
-      if (n > 3)
-        for (int k = 0; k < D; ++k) pc(id, k) = up[k] / down;
+      if (n > 3) {
+        const double r = 1.0 / down;
+        for (int k = 0; k < D; ++k) pc(id, k) = quotient(up[k], down, r);
+      }
       for (int k = 0; k < D; ++k) up[k] = 0;
       down = 0;
       n = 0;
@@ -1028,7 +1080,7 @@ __device__ __forceinline__ void plain_element4(PlainLds<4> &S, int lane, unsigne
   for (int k = 0; k < D; ++k) nrm[k] = 0;
   for_lines(S, lane, nl, ends, [&](const Line4 &l, unsigned id, bool) {
     double a[D], b[D], c[D], o[D], nv[D];
-    plain_outside(S, id, m, h, l.s, o);
+    plain_outside(S, id, m, l.s, o);
     for (int k = 0; k < D; ++k) {
       a[k] = l.s[k] - cen[k];
       b[k] = l.e[k] - cen[k];
@@ -1072,7 +1124,7 @@ __device__ __forceinline__ void plain_element3(PlainLds<3> &S, int lane, unsigne
   }
   for_lines(S, lane, nl, 0, [&](const Line4 &l, unsigned id, bool) {
     double a[D], b[D], o[D], t[D];
-    plain_outside(S, id, m, h, l.s, o);
+    plain_outside(S, id, m, l.s, o);
     for (int k = 0; k < D; ++k) {
       a[k] = l.s[k] - pm[k];
       b[k] = l.e[k] - pm[k];

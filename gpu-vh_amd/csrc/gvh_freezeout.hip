@@ -325,11 +325,12 @@ struct Spacing {
 
 // Plain cells, one per lane (gvh_cornelius.h): their elements, and the list
 // of the other surface cells for the general search.  What bounds it is
-// latency: four walks over some 28 lines, each two dependent LDS reads, and
-// the edge cuts and polygon centroids of 64 cells (40 KB in 4-D) leave one
-// wave per SIMD.  206 448 surface cubes of a 121x121x61 window: 326 us with the
-// general search of the rest, against 1590 us with a wave per cube for all;
-// 850 000 of a 201x201x101 window 1.07 against 6.14 ms.
+// latency: four walks over some 28 lines of up to 250 dependent operations
+// each, while the edge cuts and polygon centroids of 64 cells (40 KB in 4-D)
+// leave one wave per SIMD.  206 448 surface cubes of a 121x121x61 window: 255 us
+// (323 with the lines followed cube by cube and IEEE divisions in the walks),
+// against 1590 us with a wave per cube for all; 16 384 arbitrary cells, one
+// wave per CU: 70 us (100).
 template <int DIM>
 __global__ __launch_bounds__(64) void fo_plain_cells_kernel(CellSource S, long long ncells,
                                                             Spacing sp, int *__restrict__ ecnt,
@@ -352,7 +353,11 @@ __global__ __launch_bounds__(64) void fo_plain_cells_kernel(CellSource S, long l
     double v[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) v[c] = cell_corner<DIM>(S, cell, c, itl, ix, iy, iz);
-    const bool ok = corn::corner_mask<NC>(v, sp.v0, m);
+    bool ok = corn::corner_mask<NC>(v, sp.v0, m);
+    // the quotients of areas by a shared reciprocal are exact far from the
+    // ends of the exponent's range only
+#pragma unroll
+    for (int d = 4 - DIM; d < 4; ++d) ok = ok && sp.dx[d] > 1e-60 && sp.dx[d] < 1e60;
     const bool surface = m != 0u && m != (1u << NC) - 1u;
     if (surface && ok) {
       bool near = false;
