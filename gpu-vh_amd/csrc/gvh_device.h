@@ -29,6 +29,16 @@ enum { EOS_CONFORMAL = 0, EOS_WB = 1, EOS_TABLE = 2 };
 #define GVH_BLOCK 64
 #endif
 
+// Lattices of at most this many tiles of 64 cells, by the arithmetic of the
+// half-site root-finds, run their stages with several waves per tile
+// (gvh_split.hip, split_stage_fits).
+#ifndef GVH_SPLIT_MAX_TILES_FP64
+#define GVH_SPLIT_MAX_TILES_FP64 512
+#define GVH_SPLIT_MAX_TILES_FP32 1536
+#endif
+constexpr unsigned SPLIT_MAX_TILES_FP64 = GVH_SPLIT_MAX_TILES_FP64;
+constexpr unsigned SPLIT_MAX_TILES_FP32 = GVH_SPLIT_MAX_TILES_FP32;
+
 // Lattices of at least this many tiles of 64 cells run their stages in the
 // resident kernel (gvh_resident.hip).  Its blocks start with a copy of the
 // table and its 2048 (FP64) or 3072 waves end together only if each has

@@ -8,6 +8,9 @@ namespace gvh {
 bool resident_stage_fits(const StageArgs &A);
 hipError_t launch_resident_stage(const StageArgs &A, bool bulk, bool stage2, int precision,
                                  hipStream_t st);
+bool split_stage_fits(const StageArgs &A, int eos, int precision);
+hipError_t launch_split_stage(const StageArgs &A, int eos, bool bulk, bool stage2, int precision,
+                              hipStream_t st);
 
 // ------------------------------------------------------------ launch
 // Kernel arrangement of a stage (StageArgs::variant): 0 fused kernel with
@@ -25,7 +28,9 @@ hipError_t launch_resident_stage(const StageArgs &A, bool bulk, bool stage2, int
 // blocks of four rows that stage the y stencil in LDS
 // (kt_flux_kernel_ystaged); it is built for the tabulated EoS with bulk in
 // FP64 and GVH_MIXED, needs a strip height that is a multiple of 4, and runs
-// as 3 otherwise.
+// as 3 otherwise.  Arrangement 3 has two more kernels with the same
+// operations: several waves per tile for small lattices (gvh_split.hip) and
+// blocks that stay for large ones (gvh_resident.hip).
 template <int EOS, bool BULK, bool STAGE2, bool HAS_Z, bool MIXED>
 static hipError_t launch_z(const StageArgs &A, bool root64, hipStream_t st) {
   const long long ncell = (long long)A.nx * A.strip * A.nstrips * A.nz;
@@ -122,6 +127,8 @@ hipError_t launch_stage(const StageArgs &A, int eos, bool bulk, bool stage2, int
                         hipStream_t st) {
   if (A.variant == 3 && eos == EOS_TABLE && resident_stage_fits(A))
     return launch_resident_stage(A, bulk, stage2, precision, st);
+  if (A.variant == 3 && split_stage_fits(A, eos, precision))
+    return launch_split_stage(A, eos, bulk, stage2, precision, st);
   if (precision == GVH_FP64) return launch_p<false>(A, eos, bulk, stage2, false, st);
   return launch_p<true>(A, eos, bulk, stage2, precision == GVH_MIXED_F64_ROOTS, st);
 }

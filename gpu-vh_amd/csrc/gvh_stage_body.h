@@ -284,8 +284,9 @@ constexpr int BLOCK = GVH_BLOCK;
 // 45 stencil values of the nine inversion variables come from the block's
 // LDS copy of rows j-2 .. j+2 (ystage[variable][row slot][lane]) instead of
 // from memory.
+// ADD false: acc[n] = (H_b - H_f)/h + S_dir, for the caller to add.
 template <int EOS, bool BULK, int DIR, bool KEEP_STATES, int LOCK, typename R, typename PS,
-          bool YSTAGE = false, typename Tab, typename GF>
+          bool YSTAGE = false, bool ADD = true, typename Tab, typename GF>
 __device__ __forceinline__ void direction_update(const StageArgs &A, const Tab &tab, unsigned s, double ePrev,
                                                  const Guess<GF> &g, R v_s, double *acc,
                                                  const R *ystage = nullptr) {
@@ -462,7 +463,8 @@ __device__ __forceinline__ void direction_update(const StageArgs &A, const Tab &
       if (a == 1) r += Sd1;
       if (a == 2) r += Sd2;
       if (a == 3) r += Sd3;
-      acc[n * BLOCK] += (double)r * dt;
+      if constexpr (ADD) acc[n * BLOCK] += (double)r * dt;
+      else acc[n * BLOCK] = (double)r;
     }
     n0 = 8;
   }
@@ -478,7 +480,8 @@ __device__ __forceinline__ void direction_update(const StageArgs &A, const Tab &
 #pragma unroll
     for (int n = 8; n < 14; ++n) {
       const R *w = raw2[n - 8];
-      acc[n * BLOCK] += (double)flux_of(w[0], w[1], w[2], w[3], w[4]) * dt;
+      if constexpr (ADD) acc[n * BLOCK] += (double)flux_of(w[0], w[1], w[2], w[3], w[4]) * dt;
+      else acc[n * BLOCK] = (double)flux_of(w[0], w[1], w[2], w[3], w[4]);
     }
   } else {
 #pragma unroll 1
@@ -585,15 +588,18 @@ __global__ __launch_bounds__(BLOCK) void kt_source_kernel(StageArgs A) {
 // copies.  acc starts from what kt_source_kernel stored at the cell.
 // FUSED: the source terms are computed here first (one kernel per stage);
 // otherwise kt_source_kernel has stored acc = q + dt S at the cell.
+// SPLIT: the block's first wave, whose others leave the directions' rates in
+// `rates` before a barrier (kt_split_kernel).
 // YSTAGE: the thread belongs to a four-row block that staged the y stencil
 // in LDS; every thread of the block reaches the barrier before the y
 // direction, and only threads of valid cells compute (the others only
 // staged rows for their neighbours).
 template <int EOS, bool BULK, bool STAGE2, bool HAS_Z, bool FUSED, bool KEEP, int LOCK,
-          typename R, typename PS, bool YSTAGE = false, typename Tab>
+          typename R, typename PS, bool YSTAGE = false, bool SPLIT = false, typename Tab>
 __device__ __forceinline__ void stage_cell(const StageArgs &A, const Tab &tab, const CellPos &c,
                                            double *acc,
-                                           const R *ystage = nullptr) {
+                                           const R *ystage = nullptr,
+                                           const double *rates = nullptr) {
   constexpr int NV = BULK ? 15 : 14;
   const int i = c.i, j = c.j, k = c.k;
   const unsigned s = c.s;
@@ -612,7 +618,8 @@ __device__ __forceinline__ void stage_cell(const StageArgs &A, const Tab &tab, c
   using GF = typename std::conditional<LOCK != 0, flux_root_t<EOS, R, LOCK == 3>, double>::type;
   Guess<double> guess{};
   Guess<GF> fguess{};
-  if (!YSTAGE || c.valid) {
+  [[maybe_unused]] double qn_early[NV];  // SPLIT: q^n, on its way over the barrier
+  if (!(YSTAGE || SPLIT) || c.valid) {
     ut = ld_cell(u, s);
     ux = ld_cell(u + G, s);
     uy = ld_cell(u + 2 * G, s);
@@ -659,19 +666,34 @@ __device__ __forceinline__ void stage_cell(const StageArgs &A, const Tab &tab, c
     }
 
     // flux velocity of the cell itself for the directional sources (v = u/u^tau)
-    direction_update<EOS, BULK, 0, KEEP, LOCK, R, PS>(A, tab, s, e_s, fguess, div_st(R(ux), R(ut)),
-                                                       acc);
+    if constexpr (!SPLIT)
+      direction_update<EOS, BULK, 0, KEEP, LOCK, R, PS>(A, tab, s, e_s, fguess, div_st(R(ux), R(ut)),
+                                                         acc);
+    else if constexpr (STAGE2)
+#pragma unroll
+      for (int n = 0; n < NV; ++n) qn_early[n] = q_at(A.qn, n);
   }
-  if constexpr (YSTAGE) {
+  if constexpr (YSTAGE || SPLIT) {
     __syncthreads();
     if (!c.valid) return;
   }
-  direction_update<EOS, BULK, 1, KEEP, LOCK, R, PS, YSTAGE>(A, tab, s, e_s, fguess, div_st(R(uy), R(ut)),
-                                                            acc, ystage);
-  if constexpr (HAS_Z)
-    direction_update<EOS, BULK, 2, KEEP, LOCK, R, PS>(A, tab, s, e_s, fguess, div_st(R(un), R(ut)), acc);
+  if constexpr (SPLIT) {
+#pragma unroll
+    for (int n = 0; n < NV; ++n) {
+      double a = acc[n * BLOCK];
+#pragma unroll
+      for (int d = 0; d < (HAS_Z ? 3 : 2); ++d) a += rates[(d * 15 + n) * BLOCK] * A.dt;
+      if constexpr (STAGE2) a = (a + qn_early[n]) * 0.5;
+      acc[n * BLOCK] = a;
+    }
+  } else {
+    direction_update<EOS, BULK, 1, KEEP, LOCK, R, PS, YSTAGE>(A, tab, s, e_s, fguess, div_st(R(uy), R(ut)),
+                                                              acc, ystage);
+    if constexpr (HAS_Z)
+      direction_update<EOS, BULK, 2, KEEP, LOCK, R, PS>(A, tab, s, e_s, fguess, div_st(R(un), R(ut)), acc);
+  }
 
-  if constexpr (STAGE2) {
+  if constexpr (STAGE2 && !SPLIT) {
     // q^n of the convex average: all NV loads in flight together
     double qn[NV];
 #pragma unroll
