@@ -649,7 +649,7 @@ __device__ int cell_elements(Work &W, double (*cen)[D], double (*nrm)[D]) {
 //  * the polygons come in cube order, or, where a hexagon (or the 24-line
 //    pattern of two corners) makes the cell ambiguous, each time the first
 //    one that shares a square with those before it.
-// So a lane takes a whole cell: it lists its lines (a byte each), computes the
+// So a lane takes a whole cell: it lists its lines by its cubes' patterns, computes the
 // cut of each of the 32 edges once (the squares that share an edge cut it at
 // the same point) and goes over the list four times, summing in the general
 // search's order: the element equals its bit by bit.  End points are matched

@@ -11,15 +11,20 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <condition_variable>
 #include <cstddef>
+#include <memory>
+#include <mutex>
+#include <thread>
+#include <vector>
 
 namespace gvh {
 
 // One user at a time; work is ordered on the caller's stream and has ended
 // when a call returns.  The pinned memory (8 MiB, and 64 KiB for small results)
-// is allocated by the first call that needs it and freed with the object;
-// without it, below one slot, or into host memory that is pinned itself, the
-// copies are the runtime's.
+// is allocated by the first call that needs it and freed with the object, as
+// are the three threads beside the caller's; without it, below one slot, or
+// into host memory that is pinned itself, the copies are the runtime's.
 class Staging {
  public:
   Staging() = default;
@@ -35,12 +40,19 @@ class Staging {
   static constexpr int NSLOT = 8, MAX_THREADS = 4;
 
  private:
+  struct Job;
   bool ready();
+  void work();
   hipError_t pipeline(char *host, const char *dev, size_t bytes, hipStream_t st);
   char *mem_ = nullptr;  // the slots, then a flag for each
   char *small_ = nullptr;
   bool failed_ = false;
   unsigned *arrived_ = nullptr;  // per slot, blocks that have their part there
+  std::vector<std::thread> pool_;
+  std::mutex mutex_;
+  std::condition_variable wake_;
+  std::shared_ptr<Job> job_;  // the result on its way
+  bool quit_ = false;
 };
 
 }  // namespace gvh
