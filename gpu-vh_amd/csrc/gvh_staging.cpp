@@ -211,7 +211,10 @@ hipError_t Staging::pipeline(char *host, const char *dev, size_t bytes, hipStrea
 }
 
 hipError_t Staging::to_host(void *host, const void *dev, size_t bytes, hipStream_t st) {
-  if (bytes >= SLOT && bytes % 4 == 0 && !is_pinned(host) && ready()) {
+  const bool large = bytes >= SLOT && bytes % 4 == 0 && !is_pinned(host);
+  const bool pays = used_ || bytes > NSLOT * SLOT;
+  used_ = used_ || large;
+  if (large && pays && ready()) {
     try {
       return pipeline(static_cast<char *>(host), static_cast<const char *>(dev), bytes, st);
     } catch (...) {  // no memory for its bookkeeping, before anything was issued

@@ -24,7 +24,10 @@ namespace gvh {
 // when a call returns.  The pinned memory (8 MiB, and 64 KiB for small results)
 // is allocated by the first call that needs it and freed with the object, as
 // are the three threads beside the caller's; without it, below one slot, or
-// into host memory that is pinned itself, the copies are the runtime's.
+// into host memory that is pinned itself, the copies are the runtime's.  So is
+// an object's first large result, unless it is larger than the slots: to pin
+// them and to start the threads takes 0.8 ms, as much as 8 MiB take longer that
+// way, and many objects give one such result only.
 class Staging {
  public:
   Staging() = default;
@@ -46,7 +49,7 @@ class Staging {
   hipError_t pipeline(char *host, const char *dev, size_t bytes, hipStream_t st);
   char *mem_ = nullptr;  // the slots, then a flag for each
   char *small_ = nullptr;
-  bool failed_ = false;
+  bool failed_ = false, used_ = false;
   unsigned *arrived_ = nullptr;  // per slot, blocks that have their part there
   std::vector<std::thread> pool_;
   std::mutex mutex_;
